@@ -15,71 +15,9 @@
 // A row r and of B column r for its k-slice; both operands are loaded in the
 // same per-lane k order, so A/B pairing is the identity.  Result lane (g, r)
 // holds D[4g+i][r].
-#include "common.h"
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+#include "int4_dev.h"
 
 namespace {
-
-__device__ __forceinline__ v4f mfma_bf16(v4i a, v4i b, v4f c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
-}
-
-// 8 codes of one word (low nibble first along k) as bf16 (128 + q) pairs in
-// k order (0,4),(1,5),(2,6),(3,7).
-__device__ __forceinline__ v4i dequant_word(uint32_t w) {
-    return v4i{(int)((w & 0x000F000Fu) | 0x43004300u), (int)(((w >> 4) & 0x000F000Fu) | 0x43004300u),
-               (int)(((w >> 8) & 0x000F000Fu) | 0x43004300u), (int)(((w >> 12) & 0x000F000Fu) | 0x43004300u)};
-}
-
-// 8 contiguous bf16 activations reordered to the same (0,4),(1,5),(2,6),(3,7) order.
-__device__ __forceinline__ v4i permute_act(v4i a) {
-    uint32_t d0 = (uint32_t)a.x, d1 = (uint32_t)a.y, d2 = (uint32_t)a.z, d3 = (uint32_t)a.w;
-    return v4i{(int)((d0 & 0xFFFFu) | (d2 << 16)), (int)((d0 >> 16) | (d2 & 0xFFFF0000u)),
-               (int)((d1 & 0xFFFFu) | (d3 << 16)), (int)((d1 >> 16) | (d3 & 0xFFFF0000u))};
-}
-
-__device__ __forceinline__ float decode_scale(uint16_t v, bool bf16) {
-    if (bf16) return bf16_to_f32(v);
-    return (float)__builtin_bit_cast(_Float16, v);
-}
-
-__device__ __forceinline__ float load_scale(const uint16_t* p, bool bf16) { return decode_scale(*p, bf16); }
-
-constexpr uint32_t ONES_BF16 = 0x3F803F80u;
-
-struct Int4Args {
-    const uint16_t* x;
-    const uint32_t* qw;
-    const uint16_t* scales;
-    const uint32_t* qzeros;   // gptq only, may be null (zero = 8)
-    const uint16_t* aux;      // bias [N] or residual [B, N]
-    uint16_t* y;
-    uint32_t B, K, N, G;
-    int scale_bf16, finalize;
-};
-
-__device__ __forceinline__ void finalize_store(const Int4Args& A, uint32_t t, uint32_t n, float sum) {
-    // nerve/model_package_shader_selection.py:2504-2533
-    float v = sum;
-    if (A.finalize == 1) v = bf16_to_f32(A.aux[n]) + sum;
-    else if (A.finalize == 2) v = bf16_to_f32(A.aux[(uint64_t)t * A.N + n]) + round_bf16(sum);
-    A.y[(uint64_t)t * A.N + n] = (uint16_t)f32_to_bf16(v);
-}
-
-// J consecutive packed words of one qweight row (J = 1, 2 or 4).
-template <int J>
-__device__ __forceinline__ void load_words(const uint32_t* p, uint32_t (&w)[J]) {
-    if constexpr (J == 4) {
-        v4i v = *reinterpret_cast<const v4i*>(p);
-        w[0] = (uint32_t)v.x; w[1] = (uint32_t)v.y; w[2] = (uint32_t)v.z; w[3] = (uint32_t)v.w;
-    } else if constexpr (J == 2) {
-        v2i v = *reinterpret_cast<const v2i*>(p);
-        w[0] = (uint32_t)v.x; w[1] = (uint32_t)v.y;
-    } else {
-        w[0] = *p;
-    }
-}
 
 // GPTQ layout: qweight [K/8, N].  A wave owns 16 J columns (J MFMA column
 // tiles; lane r takes columns n0 + J r .. n0 + J r + J - 1 so one load feeds
@@ -290,12 +228,6 @@ __global__ __launch_bounds__(64 * KS) void int4_gptq_fixed_kernel(Int4Args A) {
 // the 16 waves' partial sums meet in LDS.
 constexpr uint32_t GEMV_MAX_M = 4;
 constexpr uint32_t GEMV_ROWS = 32;       // packed rows per wave batch (256 k)
-
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, a), __builtin_bit_cast(v2bf, b), c, false);
-}
 
 __device__ __forceinline__ float sum8_bf16(v4i v) {
     float s = 0.f;
@@ -553,13 +485,6 @@ __global__ __launch_bounds__(256) void quant_i8pp_kernel(const uint16_t* __restr
 // sum), then acc = fma(dot, s_x * s_w, acc).  Only the f32 accumulation order
 // differs from the shader (per-wave partials added in wave order).
 // ---------------------------------------------------------------------------
-struct PpArgs {
-    const uint32_t* q;          // int8 words [B, K/4], pair-packed
-    const float* s;             // [B, K/32]
-    const int32_t* sums;        // [B, K/32]
-    Int4Args L;                 // qweight, scales, aux, y, shapes
-};
-
 // Unpaired input (linear_prequant_int4_{gptq,ct}.comp.template): the int8
 // words hold columns in order, so each packed weight word becomes the signed
 // bytes (code - 8) of nibbles 0..3 and 4..7 for two v_dot4_i32_i8.
@@ -606,6 +531,248 @@ __global__ __launch_bounds__(256) void int4_pp_kernel(PpArgs P) {
         if (wave == 0 && n < N) finalize_store(A, t, n, ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]);
         __syncthreads();
     }
+}
+
+
+// ---------------------------------------------------------------------------
+// The same linears on the integer matrix cores: v_mfma_i32_16x16x32_i8
+// contracts exactly one 32-column activation block, so its int32 result is
+// the block's exact dot and each block is folded as acc_g = fma(dot, s_x,
+// acc_g), a segment of blocks that share a weight scale as acc = fma(acc_g,
+// s_w, acc).
+//
+// A wave owns 16 J columns and 16 MT tokens and the block's KS waves split the
+// blocks of K.  Operands: lane (g = l / 16, r = l % 16) supplies 8 bytes of
+// token r and of column r; the k order inside a block is free as long as both
+// agree.  Activations are read 16 bytes per lane (octets 2g, 2g+1 of 64
+// columns) and one v_permlane32_swap per dword deals them to the two blocks,
+// which leaves octet pi(g) = (0, 2, 1, 3)[g] on lane group g; the packed words
+// are read from row 4 b + pi(g) (GPTQ: J columns per load).  A word's nibbles
+// 0, 2, 4, 6 and 1, 3, 5, 7 are already the byte order of pair-packed
+// activations (column-order ones are brought into it with two v_perm); code - 8
+// per byte is ((w & 0x0f0f0f0f) + 0x78787878) ^ 0x80808080, so the block sums
+// are not needed.  The activation scales of a load batch pass through a
+// wave-private LDS slice that transposes them to result rows.
+//
+// Bound: the weight stream and, from 32 tokens on, the activation rows every
+// column tile re-reads from L2.  4096 x 14336, one token: 11.0 us a launch
+// (31.3 with a lane per column), 48 tokens: 21.7 us (about 940, tokens one by
+// one); 14336 x 4096: 13.4 and 36.6 us.
+// ---------------------------------------------------------------------------
+template <int MT, int J, int KS, int U, int BPG, bool PAIRED, bool CT>
+__global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgroups) {
+    static_assert(U % 2 == 0 && U % BPG == 0, "a batch holds whole 64-column pairs and scale segments");
+    static_assert(!CT || (J == 1 && U % 4 == 0), "CT rows are read 128 columns at a time");
+    constexpr int NV = (16 * MT * U + 63) / 64;       // activation scales per lane and batch
+    __shared__ __attribute__((aligned(16))) float xs[KS][U][16 * MT];
+    __shared__ float part[KS][J][64][4];
+    const Int4Args& A = P.L;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t g = lane >> 4, rr = lane & 15, pg = ((g & 1) << 1) | (g >> 1);
+    const uint32_t K = A.K, N = A.N, M = A.B, nblk = K / 32;
+    // Token groups fastest within an XCD's run of column tiles, so the groups
+    // of a tile read its weights through one L2.
+    const uint32_t per_xcd = gridDim.x / 8 / tgroups, seq = blockIdx.x / 8;
+    const uint32_t tile = (blockIdx.x % 8) * per_xcd + seq / tgroups;
+    const uint32_t n0 = tile * (16 * J), m0 = (seq % tgroups) * (16 * MT);
+    if (n0 >= N) return;
+    constexpr uint32_t UNIT = CT ? 4 : (BPG > 2 ? BPG : 2);
+    const uint32_t units = (nblk + UNIT - 1) / UNIT, per = (units + KS - 1) / KS;
+    const uint32_t b0 = min(nblk, wave * per * UNIT), b1 = min(nblk, b0 + per * UNIT);
+    const uint32_t col = n0 + J * rr;
+    const uint32_t ngroups = K / A.G;
+
+    struct Batch {
+        v4i a[MT][U / 2];
+        uint32_t w[U][J];
+        uint16_t sw[U / BPG][J];
+        float sx[NV];
+    };
+    const uint8_t* arow[MT];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+        arow[m] = reinterpret_cast<const uint8_t*>(P.q) + (uint64_t)min(m0 + 16 * m + rr, M - 1) * K + 16 * g;
+    // Loads past the wave's range repeat its last pair; their scales are zero.
+    auto load = [&](Batch& B, uint32_t b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if constexpr (CT) {
+                if (u % 4 == 0) {
+                    // 4 words of one block per lane, clamped into the row (K % 128 may be 64).
+                    const uint32_t bb = min(b + u + g, nblk - 1);
+                    const v4i v = *reinterpret_cast<const v4i*>(A.qw + (uint64_t)col * (K / 8) + bb * 4);
+                    B.w[u][0] = (uint32_t)v.x; B.w[u + 1][0] = (uint32_t)v.y;
+                    B.w[u + 2][0] = (uint32_t)v.z; B.w[u + 3][0] = (uint32_t)v.w;
+                }
+            } else {
+                const uint32_t bb = min(b + u, b1 - 1);
+                load_words<J>(A.qw + (uint64_t)(bb * 4 + pg) * N + col, B.w[u]);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MT; m++)
+#pragma unroll
+            for (int c = 0; c < U / 2; c++)
+                B.a[m][c] = *reinterpret_cast<const v4i*>(arow[m] + min(b + 2 * c, b1 - 2) * 32);
+#pragma unroll
+        for (int s = 0; s < U / BPG; s++) {
+            const uint32_t grp = min(b + s * BPG, b1 - 1) * 32 / A.G;
+#pragma unroll
+            for (int j = 0; j < J; j++)
+                B.sw[s][j] = CT ? A.scales[(uint64_t)(col + j) * ngroups + grp] : A.scales[(uint64_t)grp * N + col + j];
+        }
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+            const uint32_t i = v * 64 + lane, t = min(m0 + i / U, M - 1), bb = b + i % U;
+            const float s = P.s[(uint64_t)t * nblk + min(bb, b1 - 1)];
+            B.sx[v] = bb < b1 ? s : 0.0f;
+        }
+    };
+    v4f acc[MT][J];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int j = 0; j < J; j++) acc[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto contract = [&](Batch& B) __attribute__((always_inline)) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+            const uint32_t i = v * 64 + lane;
+            if (16 * MT * U % 64 == 0 || i < 16 * MT * U) xs[wave][i % U][i / U] = B.sx[v];
+        }
+        __builtin_amdgcn_wave_barrier();
+        if constexpr (CT) {
+            // Lane group g holds the 4 words of block u + g: transposed so
+            // that lane group g holds word pi(g) of each block in turn.
+#pragma unroll
+            for (int u = 0; u < U; u += 4) {
+                const auto x = __builtin_amdgcn_permlane32_swap(B.w[u][0], B.w[u + 1][0], false, false);
+                const auto y = __builtin_amdgcn_permlane32_swap(B.w[u + 2][0], B.w[u + 3][0], false, false);
+                const auto p = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
+                const auto q = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+                B.w[u][0] = p[0]; B.w[u + 1][0] = p[1]; B.w[u + 2][0] = q[0]; B.w[u + 3][0] = q[1];
+            }
+        }
+        v4f ag[MT][J];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            long bw[J];
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                const uint32_t lo = ((B.w[u][j] & 0x0f0f0f0fu) + 0x78787878u) ^ 0x80808080u;
+                const uint32_t hi = (((B.w[u][j] >> 4) & 0x0f0f0f0fu) + 0x78787878u) ^ 0x80808080u;
+                bw[j] = (long)(((uint64_t)hi << 32) | lo);
+            }
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                if (u % 2 == 0) {
+                    v4i& v = B.a[m][u / 2];
+                    if (!PAIRED) {
+                        const uint32_t e0 = __builtin_amdgcn_perm((uint32_t)v.y, (uint32_t)v.x, 0x06040200u);
+                        const uint32_t o0 = __builtin_amdgcn_perm((uint32_t)v.y, (uint32_t)v.x, 0x07050301u);
+                        const uint32_t e1 = __builtin_amdgcn_perm((uint32_t)v.w, (uint32_t)v.z, 0x06040200u);
+                        const uint32_t o1 = __builtin_amdgcn_perm((uint32_t)v.w, (uint32_t)v.z, 0x07050301u);
+                        v = v4i{(int)e0, (int)o0, (int)e1, (int)o1};
+                    }
+                    const auto x = __builtin_amdgcn_permlane32_swap((uint32_t)v.x, (uint32_t)v.z, false, false);
+                    const auto y = __builtin_amdgcn_permlane32_swap((uint32_t)v.y, (uint32_t)v.w, false, false);
+                    v = v4i{(int)x[0], (int)y[0], (int)x[1], (int)y[1]};
+                }
+                const v4i& v = B.a[m][u / 2];
+                const uint32_t a0 = (uint32_t)(u % 2 ? v.z : v.x), a1 = (uint32_t)(u % 2 ? v.w : v.y);
+                const long av = (long)(((uint64_t)a1 << 32) | a0);
+                const v4f sx = *reinterpret_cast<const v4f*>(&xs[wave][u][16 * m + 4 * g]);
+#pragma unroll
+                for (int j = 0; j < J; j++) {
+                    const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bw[j], v4i{0, 0, 0, 0}, 0, 0, 0);
+                    if (u % BPG == 0) ag[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int i = 0; i < 4; i++) ag[m][j][i] = fmaf((float)d[i], sx[i], ag[m][j][i]);
+                    if (u % BPG == BPG - 1) {
+                        const float sw = decode_scale(B.sw[u / BPG][j], A.scale_bf16);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[m][j][i] = fmaf(ag[m][j][i], sw, acc[m][j][i]);
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    if (b0 < b1) {
+        Batch p, q;
+        load(p, b0);
+        for (uint32_t b = b0; b < b1; b += 2 * U) {
+            const bool two = b + U < b1;
+            if (two) load(q, b + U);
+            contract(p);
+            if (!two) break;
+            if (b + 2 * U < b1) load(p, b + 2 * U);
+            contract(q);
+        }
+    }
+    // The waves' partial sums meet in LDS one token tile at a time and are
+    // added in wave order.
+#pragma unroll
+    for (int m = 0; m < MT; m++) {
+        if (m0 + 16 * m >= M) break;
+#pragma unroll
+        for (int j = 0; j < J; j++) *reinterpret_cast<v4f*>(&part[wave][j][lane][0]) = acc[m][j];
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < 256 * J; i += 64 * KS) {
+            const uint32_t t = i / (16 * J), c = i % (16 * J), tt = m0 + 16 * m + t;
+            if (tt >= M) break;
+            const uint32_t l = (t / 4) * 16 + c / J;
+            float v = part[0][c % J][l][t % 4];
+#pragma unroll
+            for (int w = 1; w < KS; w++) v += part[w][c % J][l][t % 4];
+            finalize_store(A, tt, n0 + c, v);
+        }
+        __syncthreads();
+    }
+}
+
+// SEG: blocks per scale segment (a divisor of the group's blocks), at most a
+// batch.
+template <int MT, int J, int KS, int U, int SEG>
+void launch_i8_form(const PpArgs& P, bool paired, bool ct, hipStream_t st) {
+    constexpr int BPG = SEG < U ? SEG : U;
+    const uint32_t tg = (P.L.B + 16 * MT - 1) / (16 * MT), tiles = P.L.N / (16 * J);
+    const uint32_t grid = (tiles + 7) / 8 * 8 * tg;
+    if (paired) int4_i8_kernel<MT, J, KS, U, BPG, true, false><<<grid, 64 * KS, 0, st>>>(P, tg);
+    else if (!ct) int4_i8_kernel<MT, J, KS, U, BPG, false, false><<<grid, 64 * KS, 0, st>>>(P, tg);
+    else if constexpr (J == 1) int4_i8_kernel<MT, J, KS, U, BPG, false, true><<<grid, 64 * KS, 0, st>>>(P, tg);
+}
+
+template <int SEG>
+void launch_i8_shape(const PpArgs& P, bool paired, bool ct, uint32_t j, hipStream_t st) {
+    const uint32_t mt = (P.L.B + 15) / 16;
+    if (j == 4) {
+        if (mt == 1) launch_i8_form<1, 4, 8, 8, SEG>(P, paired, ct, st);
+        else if (mt == 2) launch_i8_form<2, 4, 8, 4, SEG>(P, paired, ct, st);
+        else launch_i8_form<3, 4, 8, 2, SEG>(P, paired, ct, st);
+    } else {
+        if (mt == 1) launch_i8_form<1, 1, 8, 16, SEG>(P, paired, ct, st);
+        else if (mt == 2) launch_i8_form<2, 1, 8, 8, SEG>(P, paired, ct, st);
+        else launch_i8_form<4, 1, 8, 4, SEG>(P, paired, ct, st);
+    }
+}
+
+// Launches the matrix-core form when the shape and alignment allow its 16-byte
+// loads (whole 16-column tiles; whole 64-column activation pairs, 128 columns
+// for CT rows); false otherwise (int4_pp_kernel takes every other shape).
+// 64-column tiles (16 bytes a lane) where they fill more than half of the CUs,
+// else 16-column ones: at N = 4096 the 64 wide tiles would stream 29 MB through
+// 64 CUs, and a CU takes in about 27 GB/s.
+bool launch_i8(const PpArgs& P, bool paired, bool ct, int cus, hipStream_t st) {
+    const Int4Args& A = P.L;
+    if (A.N % 16 || A.K % 64 || ((uintptr_t)P.q & 15) || ((uintptr_t)A.qw & 15)) return false;
+    if (ct && A.K % 128) return false;
+    const uint32_t tg = (A.B + 63) / 64;
+    const uint32_t j = !ct && A.N % 64 == 0 && A.N / 64 * tg * 2 > (uint32_t)cus ? 4 : 1;
+    const uint32_t bpg = A.G % 128 == 0 ? 4 : A.G % 64 == 0 ? 2 : 1;
+    if (bpg == 4) launch_i8_shape<4>(P, paired, ct, j, st);
+    else if (bpg == 2) launch_i8_shape<2>(P, paired, ct, j, st);
+    else launch_i8_shape<1>(P, paired, ct, j, st);
+    return true;
 }
 
 }  // namespace
@@ -784,6 +951,7 @@ extern "C" nerve_hip_status nerve_hip_int4_linear_pairpacked(nerve_hip_ctx* ctx,
     P.L.finalize = s.op;
     const uint32_t grid = (s.out + 63) / 64;
     hipStream_t strm = (hipStream_t)stream;
+    if (launch_i8(P, paired, s.layout == 1, ctx->cu_count, strm)) return nh::check_launch("int4_linear_prequant");
     if (paired) int4_pp_kernel<true, false><<<grid, 256, 0, strm>>>(P);
     else if (s.layout == 0) int4_pp_kernel<false, false><<<grid, 256, 0, strm>>>(P);
     else int4_pp_kernel<false, true><<<grid, 256, 0, strm>>>(P);

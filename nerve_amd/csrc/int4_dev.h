@@ -1,0 +1,91 @@
+// Shared pieces of the INT4 linears: code expansion, scale decoding, the
+// kernel arguments and the finalizing store.
+#pragma once
+
+#include "common.h"
+
+namespace nh {
+
+struct Int4Args {
+    const uint16_t* x;
+    const uint32_t* qw;
+    const uint16_t* scales;
+    const uint32_t* qzeros;   // gptq only, may be null (zero = 8)
+    const uint16_t* aux;      // bias [N] or residual [B, N]
+    uint16_t* y;
+    uint32_t B, K, N, G;
+    int scale_bf16, finalize;
+};
+
+struct PpArgs {
+    const uint32_t* q;          // int8 words [B, K/4], pair-packed
+    const float* s;             // [B, K/32]
+    const int32_t* sums;        // [B, K/32]
+    Int4Args L;                 // qweight, scales, aux, y, shapes
+};
+
+}  // namespace nh
+
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+namespace {
+
+using nh::Int4Args;
+using nh::PpArgs;
+
+__device__ __forceinline__ v4f mfma_bf16(v4i a, v4i b, v4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+}
+
+// 8 codes of one word (low nibble first along k) as bf16 (128 + q) pairs in
+// k order (0,4),(1,5),(2,6),(3,7).
+__device__ __forceinline__ v4i dequant_word(uint32_t w) {
+    return v4i{(int)((w & 0x000F000Fu) | 0x43004300u), (int)(((w >> 4) & 0x000F000Fu) | 0x43004300u),
+               (int)(((w >> 8) & 0x000F000Fu) | 0x43004300u), (int)(((w >> 12) & 0x000F000Fu) | 0x43004300u)};
+}
+
+// 8 contiguous bf16 activations reordered to the same (0,4),(1,5),(2,6),(3,7) order.
+__device__ __forceinline__ v4i permute_act(v4i a) {
+    uint32_t d0 = (uint32_t)a.x, d1 = (uint32_t)a.y, d2 = (uint32_t)a.z, d3 = (uint32_t)a.w;
+    return v4i{(int)((d0 & 0xFFFFu) | (d2 << 16)), (int)((d0 >> 16) | (d2 & 0xFFFF0000u)),
+               (int)((d1 & 0xFFFFu) | (d3 << 16)), (int)((d1 >> 16) | (d3 & 0xFFFF0000u))};
+}
+
+__device__ __forceinline__ float decode_scale(uint16_t v, bool bf16) {
+    if (bf16) return bf16_to_f32(v);
+    return (float)__builtin_bit_cast(_Float16, v);
+}
+
+__device__ __forceinline__ float load_scale(const uint16_t* p, bool bf16) { return decode_scale(*p, bf16); }
+
+constexpr uint32_t ONES_BF16 = 0x3F803F80u;
+
+__device__ __forceinline__ void finalize_store(const Int4Args& A, uint32_t t, uint32_t n, float sum) {
+    // nerve/model_package_shader_selection.py:2504-2533
+    float v = sum;
+    if (A.finalize == 1) v = bf16_to_f32(A.aux[n]) + sum;
+    else if (A.finalize == 2) v = bf16_to_f32(A.aux[(uint64_t)t * A.N + n]) + round_bf16(sum);
+    A.y[(uint64_t)t * A.N + n] = (uint16_t)f32_to_bf16(v);
+}
+
+// J consecutive packed words of one qweight row (J = 1, 2 or 4).
+template <int J>
+__device__ __forceinline__ void load_words(const uint32_t* p, uint32_t (&w)[J]) {
+    if constexpr (J == 4) {
+        v4i v = *reinterpret_cast<const v4i*>(p);
+        w[0] = (uint32_t)v.x; w[1] = (uint32_t)v.y; w[2] = (uint32_t)v.z; w[3] = (uint32_t)v.w;
+    } else if constexpr (J == 2) {
+        v2i v = *reinterpret_cast<const v2i*>(p);
+        w[0] = (uint32_t)v.x; w[1] = (uint32_t)v.y;
+    } else {
+        w[0] = *p;
+    }
+}
+
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, a), __builtin_bit_cast(v2bf, b), c, false);
+}
+
+}  // namespace

@@ -175,3 +175,43 @@ def test_int4_linear_prequant_unpaired(ctx, dev, M, K, N, G, layout, finalize):
     ok, worst, exact = bf16_close(to_np(y, np.uint16), ref, atol=linear_atol(x, gptq_dequant(d), finalize),
                                   name="prequant unpaired")
     assert ok and exact > 0.9, (worst, exact)
+
+
+# The matrix-core form's edges: one 64-column pair (K = 64), K that is not a
+# multiple of 128, scale segments of 1, 2 and 4 blocks (G = 96 and 160 fall
+# back to one), waves with no blocks, both column-tile widths (N >= 8256 takes
+# 64 columns), N = 16 and 80, and every token-tile count with remainders.
+@pytest.mark.parametrize("kind", ["paired", "gptq", "ct"])
+@pytest.mark.parametrize("M,K,N,G", [(1, 64, 16, 32), (2, 2880, 80, 64), (5, 384, 48, 96), (16, 640, 320, 160),
+                                     (17, 1024, 8256, 256), (33, 256, 8320, 128), (49, 2880, 8256, 64),
+                                     (65, 512, 80, 32), (130, 384, 4160, 128)])
+def test_int4_linear_prequant_tiles(ctx, dev, kind, M, K, N, G):
+    import torch
+
+    rng = np.random.default_rng(M + K + N + G)
+    d = wl.int4_gptq(rng, K, N, G, True)
+    finalize = M % 3
+    qw, sc = _ct_layout(d, K, N) if kind == "ct" else (d["qweight"], d["scales"])
+    sc_bits = wl.f32_to_bf16_bits(sc.astype(np.float32)) if M % 2 else sc.view(np.uint16)
+    x = wl.bf16_normal(rng, (M, K))
+    aux = wl.bf16_normal(rng, (M, N)) if finalize == 2 else wl.bf16_normal(rng, (N,)) if finalize == 1 else None
+    q, s, sums = _quant(ctx, dev, x) if kind == "paired" else (*_quant_unpaired(ctx, dev, x), None)
+    # Rows past M stay untouched.
+    y = torch.full((M + 1, N), 0x7FC0, dtype=torch.int16, device=dev)
+    op = ["linear", "linear_bias", "linear_residual"][finalize]
+    spec = (f"{op}_prequant{'_pairpacked' if kind == 'paired' else ''}_batch16_int4_{'ct' if kind == 'ct' else 'gptq'}"
+            f"_s{'bf16' if M % 2 else 'f16'}_g{G}_{K}x{N}.comp")
+    ctx.int4_linear_pairpacked(spec, q, s, sums, to_dev(qw, dev), to_dev(sc_bits, dev),
+                               None if aux is None else to_dev(aux, dev), y, M)
+    got = to_np(y, np.uint16)
+    assert np.all(got[M] == 0x7FC0)
+    if kind == "paired":
+        qr, sr, sumr = oracle.quantize_i8_pairpacked(x)
+        ref = oracle.int4_linear_pairpacked(qr, sr, sumr, qw, sc_bits, G, scale_bf16=bool(M % 2), finalize=finalize,
+                                            aux=aux)
+    else:
+        qr, sr = oracle.quantize_i8(x)
+        ref = oracle.int4_linear_prequant(kind, qr, sr, qw, sc_bits, G, scale_bf16=bool(M % 2), finalize=finalize,
+                                          aux=aux)
+    ok, worst, exact = bf16_close(got[:M], ref, atol=linear_atol(x, gptq_dequant(d), finalize), name="prequant tiles")
+    assert ok and exact > 0.9, (worst, exact)
