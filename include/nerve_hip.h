@@ -358,7 +358,9 @@ nerve_hip_status nerve_hip_int4_moe_down(nerve_hip_ctx* ctx, const char* spec, c
  * comp.template:85-233; grammar nerve/model_package_shader_templates.py:
  * 3148-3215): per group, the bf16 MFMA sum of (code - 8) x, then
  * fma(group_sum, scale, acc), any batch_width (the CT layout with group % 128
- * != 0 returns NERVE_HIP_UNSUPPORTED). */
+ * != 0 returns NERVE_HIP_UNSUPPORTED).  More than 16 rows may split K over the
+ * launch: the partial sums use a part of the context's device memory allocated
+ * by nerve_hip_open (32 MiB; no call grows it, so a first call may be captured). */
 nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char* spec,
                                        const void* x_bf16, const void* qweight,
                                        const void* scales, const void* zeros,

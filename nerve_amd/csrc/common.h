@@ -130,12 +130,16 @@ struct nerve_hip_ctx {
     size_t workspace_bytes;
     void* static_scratch;         // device address of this device's static scratch array
     uint32_t* sync_words;         // arrival counters of single-launch reductions (zeroed at open)
+    void* split;                  // split-K partial sums, nh::kSplitBytes (allocated at open: no call grows it)
 };
 
 namespace nh {
 
 // Size of the file-scope device array behind the no-allocation entry point.
 constexpr size_t kStaticScratchBytes = 4u << 20;
+
+// Size of a context's split-K scratch.
+constexpr size_t kSplitBytes = 32u << 20;
 
 nerve_hip_status fail(nerve_hip_status code, const std::string& msg);
 nerve_hip_status ok();

@@ -433,7 +433,14 @@ nerve_hip_status nerve_hip_open(int device_ordinal, nerve_hip_ctx** out) {
         (void)hipFree(sync_words);
         return nh::fail(NERVE_HIP_DEVICE_ERROR, std::string("hipMemset: ") + hipGetErrorString(e));
     }
+    void* split = nullptr;
+    e = hipMalloc(&split, nh::kSplitBytes);
+    if (e != hipSuccess) {
+        (void)hipFree(sync_words);
+        return nh::fail(NERVE_HIP_OUT_OF_MEMORY, std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
     nerve_hip_ctx* ctx = new nerve_hip_ctx();
+    ctx->split = split;
     ctx->device = device_ordinal;
     ctx->sync_words = sync_words;
     ctx->cu_count = prop.multiProcessorCount;
@@ -501,6 +508,7 @@ void nerve_hip_close(nerve_hip_ctx* ctx) {
     (void)hipDeviceSynchronize();
     if (ctx->workspace) (void)hipFree(ctx->workspace);
     if (ctx->sync_words) (void)hipFree(ctx->sync_words);
+    if (ctx->split) (void)hipFree(ctx->split);
     delete ctx;
 }
 

@@ -554,10 +554,10 @@ __global__ __launch_bounds__(256) void int4_pp_kernel(PpArgs P) {
 // are not needed.  The activation scales of a load batch pass through a
 // wave-private LDS slice that transposes them to result rows.
 //
-// Bound: the weight stream and, from 32 tokens on, the activation rows every
-// column tile re-reads from L2.  4096 x 14336, one token: 11.0 us a launch
-// (31.3 with a lane per column), 48 tokens: 21.7 us (about 940, tokens one by
-// one); 14336 x 4096: 13.4 and 36.6 us.
+// Bound: the weight stream and, from about 32 tokens on, the activation rows
+// every column tile re-reads from L2.  One token of 4096 x 14336: 11.0 us a
+// launch (31.3 with a lane per column), of 14336 x 4096 13.4 us; a feed-forward
+// of 30 tokens 1782 -> 62 us.
 // ---------------------------------------------------------------------------
 template <int MT, int J, int KS, int U, int BPG, bool PAIRED, bool CT>
 __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgroups) {
@@ -747,12 +747,10 @@ void launch_i8_shape(const PpArgs& P, bool paired, bool ct, uint32_t j, hipStrea
     const uint32_t mt = (P.L.B + 15) / 16;
     if (j == 4) {
         if (mt == 1) launch_i8_form<1, 4, 8, 8, SEG>(P, paired, ct, st);
-        else if (mt == 2) launch_i8_form<2, 4, 8, 4, SEG>(P, paired, ct, st);
-        else launch_i8_form<3, 4, 8, 2, SEG>(P, paired, ct, st);
+        else launch_i8_form<2, 4, 8, 4, SEG>(P, paired, ct, st);
     } else {
         if (mt == 1) launch_i8_form<1, 1, 8, 16, SEG>(P, paired, ct, st);
-        else if (mt == 2) launch_i8_form<2, 1, 8, 8, SEG>(P, paired, ct, st);
-        else launch_i8_form<4, 1, 8, 4, SEG>(P, paired, ct, st);
+        else launch_i8_form<2, 1, 8, 8, SEG>(P, paired, ct, st);
     }
 }
 
@@ -766,7 +764,7 @@ bool launch_i8(const PpArgs& P, bool paired, bool ct, int cus, hipStream_t st) {
     const Int4Args& A = P.L;
     if (A.N % 16 || A.K % 64 || ((uintptr_t)P.q & 15) || ((uintptr_t)A.qw & 15)) return false;
     if (ct && A.K % 128) return false;
-    const uint32_t tg = (A.B + 63) / 64;
+    const uint32_t tg = (A.B + 31) / 32;
     const uint32_t j = !ct && A.N % 64 == 0 && A.N / 64 * tg * 2 > (uint32_t)cus ? 4 : 1;
     const uint32_t bpg = A.G % 128 == 0 ? 4 : A.G % 64 == 0 ? 2 : 1;
     if (bpg == 4) launch_i8_shape<4>(P, paired, ct, j, st);
@@ -808,6 +806,15 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
     A.scale_bf16 = s.scale_bf16;
     A.finalize = s.op;
     hipStream_t strm = (hipStream_t)stream;
+    // More than 16 rows: the tiled split-K form, which expands the weights once
+    // per 64 rows instead of once per 16.  The 16-row kernels stay where one
+    // round of their blocks covers a GPTQ linear with a short K (64 rows of
+    // 4096 x 4096: 10.1 against 15.1 us; of 14336 x 4096: 25.9 against 20.0).
+    const bool one_round = s.layout == 0 && A.N % 64 == 0 && A.K <= 6144 &&
+                           (uint64_t)(A.N / 64) * ((batch_width + 15) / 16) <= (uint64_t)ctx->cu_count;
+    if (batch_width > 16 && !one_round && !(s.layout == 1 && (zeros || A.G % 128)) &&
+        nh::int4_gemm(ctx, A, nullptr, false, s.layout == 1, strm))
+        return nh::check_launch("int4_linear_gemm");
     if (s.layout == 0) {
         if (A.N % 16) return nh::fail(NERVE_HIP_UNSUPPORTED, "GPTQ INT4 kernel needs N % 16 == 0");
         if (zeros && A.N % 8) return nh::fail(NERVE_HIP_INVALID_ARGUMENT, "qzeros need N % 8 == 0");
@@ -951,6 +958,10 @@ extern "C" nerve_hip_status nerve_hip_int4_linear_pairpacked(nerve_hip_ctx* ctx,
     P.L.finalize = s.op;
     const uint32_t grid = (s.out + 63) / 64;
     hipStream_t strm = (hipStream_t)stream;
+    // More than 32 rows: the tiled split-K form (48 rows through a 4096 x 14336
+    // feed-forward: 79 us against 88; 30 rows: 66 against 62).
+    if (batch_width > 32 && nh::int4_gemm(ctx, P.L, &P, paired, s.layout == 1, strm))
+        return nh::check_launch("int4_linear_prequant");
     if (launch_i8(P, paired, s.layout == 1, ctx->cu_count, strm)) return nh::check_launch("int4_linear_prequant");
     if (paired) int4_pp_kernel<true, false><<<grid, 256, 0, strm>>>(P);
     else if (s.layout == 0) int4_pp_kernel<false, false><<<grid, 256, 0, strm>>>(P);

@@ -44,6 +44,19 @@ __device__ __forceinline__ v4i dequant_word(uint32_t w) {
                (int)(((w >> 8) & 0x000F000Fu) | 0x43004300u), (int)(((w >> 12) & 0x000F000Fu) | 0x43004300u)};
 }
 
+// The same with the exponent bits in a vector register (pair_exponent()): mask
+// and exponent are then one v_and_or_b32 (an instruction takes no literal there
+// and one scalar operand at most), 7 instructions a word instead of 11.
+__device__ __forceinline__ uint32_t pair_exponent() {
+    uint32_t e;
+    asm("v_mov_b32 %0, 0x43004300" : "=v"(e));
+    return e;
+}
+__device__ __forceinline__ v4i dequant_word(uint32_t w, uint32_t e) {
+    return v4i{(int)((w & 0x000F000Fu) | e), (int)(((w >> 4) & 0x000F000Fu) | e),
+               (int)(((w >> 8) & 0x000F000Fu) | e), (int)(((w >> 12) & 0x000F000Fu) | e)};
+}
+
 // 8 contiguous bf16 activations reordered to the same (0,4),(1,5),(2,6),(3,7) order.
 __device__ __forceinline__ v4i permute_act(v4i a) {
     uint32_t d0 = (uint32_t)a.x, d1 = (uint32_t)a.y, d2 = (uint32_t)a.z, d3 = (uint32_t)a.w;
@@ -89,3 +102,12 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
 }
 
 }  // namespace
+
+namespace nh {
+
+// Tiled split-K form for more than 16 rows (int4_gemm.hip): launches and
+// returns true when the shape and alignment allow its loads, else false.
+// `i8` is null for bf16 activations.
+bool int4_gemm(const nerve_hip_ctx* ctx, const Int4Args& A, const PpArgs* i8, bool paired, bool ct, hipStream_t st);
+
+}  // namespace nh

@@ -256,3 +256,36 @@ def test_int4_cooperative_batch64(ctx, dev, B, layout, G, finalize):
     ref = oracle.int4_linear(layout, x, qw, sc.view(np.uint16), G, finalize=finalize, aux=aux)
     ok, worst, exact = bf16_close(y, ref, atol=linear_atol(x, gptq_dequant(d), finalize), name="int4 cooperative")
     assert ok and exact > 0.9, (worst, exact)
+
+
+# The tiled split-K form (more than 16 rows): row tiles 1..4 with remainders,
+# column tiles cut at 16 and at 256, K tails of half a stage, scale segments of
+# 1, 2 and 4 blocks (G = 96 falls back to one), with and without zero points,
+# one split and several, and rows past M left alone.
+@pytest.mark.parametrize("layout,M,K,N,G,asym", [
+    ("gptq", 17, 256, 80, 128, True), ("gptq", 33, 2880, 272, 64, True), ("gptq", 49, 2880, 528, 32, False),
+    ("gptq", 65, 384, 48, 96, True), ("gptq", 130, 8192, 64, 256, False), ("gptq", 200, 1088, 1040, 64, False),
+    ("gptq", 257, 128, 16384, 128, True), ("ct", 17, 128, 16, 128, False), ("ct", 48, 4096, 272, 128, False),
+    ("ct", 100, 768, 1040, 256, False), ("ct", 301, 384, 528, 128, False)])
+def test_int4_linear_tiles(ctx, dev, layout, M, K, N, G, asym):
+    rng = np.random.default_rng(M + K + N + G)
+    d = wl.int4_gptq(rng, K, N, G, not asym)
+    finalize = M % 3
+    qw, sc = (d["qweight"], d["scales"]) if layout == "gptq" else _ct_from_gptq(d, K, N, G)
+    bf = M % 2 == 0
+    sc = wl.f32_to_bf16_bits(sc.astype(np.float32)) if bf else sc.view(np.uint16)
+    x = wl.bf16_normal(rng, (M, K))
+    aux = wl.bf16_normal(rng, (M, N)) if finalize == 2 else wl.bf16_normal(rng, (N,)) if finalize == 1 else None
+    op = ["linear", "linear_bias", "linear_residual"][finalize]
+    spec = f"{op}_batch16_int4_{layout}_s{'bf16' if bf else 'f16'}_g{G}_{K}x{N}.comp"
+    torch = _torch()
+    y = torch.full((M + 1, N), 0x7FC0, dtype=torch.int16, device=dev)
+    zeros = d["qzeros"] if asym else None
+    ctx.int4_linear(spec, to_dev(x, dev), to_dev(qw, dev), to_dev(np.ascontiguousarray(sc), dev),
+                    None if zeros is None else to_dev(zeros, dev), None if aux is None else to_dev(aux, dev), y, M)
+    got = to_np(y, np.uint16)
+    assert np.all(got[M] == 0x7FC0)
+    ref = oracle.int4_linear(layout, x, qw, np.ascontiguousarray(sc), G, scale_bf16=bf, zeros=zeros,
+                             finalize=finalize, aux=aux)
+    ok, worst, exact = bf16_close(got[:M], ref, atol=linear_atol(x, gptq_dequant(d), finalize), name="int4 tiles")
+    assert ok and exact > 0.9, (worst, exact)
