@@ -91,6 +91,7 @@ __global__ __launch_bounds__(64 * RL_WAVES) void router_linear_kernel(const uint
     router_tile(x, W, B, H, E, blockIdx.x * 16, blockIdx.y * 16, threadIdx.x >> 6, true, part, logits, E);
 }
 
+// E > 256: one wave per token, the rounds over LDS.
 __global__ __launch_bounds__(64) void topk_kernel(const uint16_t* __restrict__ logits, const void* __restrict__ bias,
                                                   uint32_t* __restrict__ routes, uint32_t* __restrict__ telemetry,
                                                   uint32_t B, TopkParams P) {
@@ -101,12 +102,28 @@ __global__ __launch_bounds__(64) void topk_kernel(const uint16_t* __restrict__ l
     __shared__ uint32_t sel_total, res_total;
     const uint32_t b = blockIdx.x;
     if (b >= B) return;
-    if (P.mode == 0 && P.E <= 64) {
-        topk_token_fast(logits + (uint64_t)b * P.E, bias, routes, telemetry, b, true, P, nullptr, sh);
-        return;
-    }
     TopkScratch S{sh, reinterpret_cast<uint32_t*>(sh + P.E), top, wts, &smax_sh, &sden_sh, &sel_total, &res_total};
     topk_token(logits + (uint64_t)b * P.E, bias, routes, telemetry, b, true, P, S);
+}
+
+// E <= 256: one wave per token.  With lds_tel the block counts in LDS (T words, dynamic) and adds its nonzero
+// counts to the telemetry once: popular experts' counters would otherwise take
+// one device atomic per token, all on a few addresses.
+__global__ __launch_bounds__(1024) void topk_wave_kernel(const uint16_t* __restrict__ logits,
+                                                         const void* __restrict__ bias, uint32_t* __restrict__ routes,
+                                                         uint32_t* __restrict__ telemetry, uint32_t B,
+                                                         uint32_t lds_tel, TopkParams P) {
+    extern __shared__ uint32_t tel[];
+    __shared__ __attribute__((aligned(16))) float s_sh[16][64];
+    const uint32_t wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    for (uint32_t i = threadIdx.x; i < lds_tel; i += blockDim.x) tel[i] = 0;
+    if (lds_tel) __syncthreads();
+    const uint32_t b = blockIdx.x * nw + wave;
+    if (b < B) topk_wave(logits + (uint64_t)b * P.E, bias, routes, lds_tel ? tel : telemetry, b, P, lds_tel != 0, s_sh[wave]);
+    if (!lds_tel) return;
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < lds_tel; i += blockDim.x)
+        if (tel[i]) __hip_atomic_fetch_add(&telemetry[i], tel[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __global__ __launch_bounds__(1024) void compact_kernel(CompactArgs A) {
@@ -183,7 +200,7 @@ __device__ __forceinline__ void route_quant_rows(const QuantArgs& Q, uint32_t w,
     }
 }
 
-constexpr uint32_t FR_LDS_TELEMETRY = 4096;   // telemetry arrays up to this size are counted in LDS
+constexpr uint32_t FR_LDS_TELEMETRY = 16384;   // telemetry arrays up to this size are counted in LDS
 
 __device__ __forceinline__ void coherent_store_f(float* p, float v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -195,11 +212,6 @@ __device__ __forceinline__ float coherent_load_f(const float* p) {
 __global__ __launch_bounds__(1024) void route_fused_kernel(FusedRouteArgs F) {
     __shared__ uint16_t lg[FR_MAX_TOKENS * FR_MAX_EXPERTS];
     __shared__ __attribute__((aligned(16))) float t_raw[16][FR_MAX_EXPERTS];
-    __shared__ uint32_t t_sel[16][FR_MAX_EXPERTS];
-    __shared__ uint32_t t_top[16][128];
-    __shared__ float t_wts[16][128];
-    __shared__ float t_f[16][2];
-    __shared__ uint32_t t_u[16][2];
     __shared__ uint32_t rl[1024];                  // route words, [B][total_sel]
     __shared__ uint32_t tel[FR_LDS_TELEMETRY];
     __shared__ uint32_t wave_tot[16];
@@ -301,17 +313,8 @@ __global__ __launch_bounds__(1024) void route_fused_kernel(FusedRouteArgs F) {
             if (b0 + 2 * wave < B)
                 topk_pair32(lg, E, F.bias, rl, telp, b0 + 2 * wave, B, F.P, t_raw[wave], tel_in_lds);
     } else {
-        TopkScratch S{t_raw[wave], t_sel[wave], t_top[wave], t_wts[wave], &t_f[wave][0], &t_f[wave][1],
-                      &t_u[wave][0], &t_u[wave][1]};
-        const bool fast = F.P.mode == 0 && E <= 64;
-        for (uint32_t b0 = 0; b0 < B; b0 += 16) {
-            const uint32_t b = b0 + wave;
-            if (fast) {
-                if (b < B)   // wave-level only, like topk_pair32
-                    topk_token_fast(lg + b * E, F.bias, rl, telp, b, true, F.P, tel_in_lds ? tel : nullptr, t_raw[wave]);
-            }
-            else topk_token(lg + (b < B ? b : 0) * E, F.bias, rl, telp, b, b < B, F.P, S, tel_in_lds ? tel : nullptr);
-        }
+        // Waves work on their tokens alone (nothing synchronizes the block).
+        for (uint32_t t = wave; t < B; t += 16) topk_wave(lg + t * E, F.bias, rl, telp, t, F.P, tel_in_lds, t_raw[wave]);
     }
     __syncthreads();
     CompactArgs C = F.C;
@@ -409,10 +412,22 @@ nerve_hip_status nerve_hip_moe_router_topk(nerve_hip_ctx* ctx, const char* spec,
     P.softcap = ts.softcap;
     P.routed_scale = ts.routed_scale;
     P.always_weight = ts.always_weight;
-    size_t lds = (size_t)(ts.experts + 3) / 4 * 4 * 8;   // >= E floats rounded up to float4s, twice
-    topk_kernel<<<batch_width, 64, lds, (hipStream_t)stream>>>(static_cast<const uint16_t*>(logits_bf16), bias,
-                                                               static_cast<uint32_t*>(routes_u32),
-                                                               static_cast<uint32_t*>(telemetry_u32), batch_width, P);
+    hipStream_t strm = (hipStream_t)stream;
+    const uint16_t* lg = static_cast<const uint16_t*>(logits_bf16);
+    uint32_t* rt = static_cast<uint32_t*>(routes_u32);
+    uint32_t* tel = static_cast<uint32_t*>(telemetry_u32);
+    if (ts.experts <= 256) {
+        // From 256 tokens on a block takes 16 tokens, so that its LDS counts
+        // are worth their flush (up to 60 KiB of counters).
+        const uint32_t res = ts.experts + (ts.mode == 1 ? ts.always_count : 0u), T = res + res * (res - 1) / 2;
+        const bool lds_tel = tel && batch_width >= 256 && T <= 15360;
+        const uint32_t nw = lds_tel ? 16 : 4;
+        topk_wave_kernel<<<(batch_width + nw - 1) / nw, 64 * nw, lds_tel ? T * 4 : 0, strm>>>(
+            lg, bias, rt, tel, batch_width, lds_tel ? T : 0u, P);
+    } else {
+        const size_t lds = (size_t)(ts.experts + 3) / 4 * 4 * 8;   // >= E floats rounded up to float4s, twice
+        topk_kernel<<<batch_width, 64, lds, strm>>>(lg, bias, rt, tel, batch_width, P);
+    }
     return nh::check_launch("moe_router_topk");
 }
 

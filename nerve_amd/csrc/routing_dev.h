@@ -421,6 +421,165 @@ __device__ void topk_pair32(const uint16_t* lg, uint32_t stride, const void* bia
     }
 }
 
+// Wave max with the same tree in every lane (DPP row operations and row swaps).
+__device__ __forceinline__ float wave_max64(float v) {
+    v = fmaxf(v, dpp_f32<0xB1>(v));
+    v = fmaxf(v, dpp_f32<0x4E>(v));
+    v = fmaxf(v, dpp_f32<0x141>(v));
+    v = fmaxf(v, dpp_f32<0x140>(v));
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
+}
+
+// Top-k of one token by one wave with the experts in registers (lane l holds
+// experts l, l + 64, ...; E <= 64 R), both grammars: the result of
+// topk_token's arg-max rounds, bit for bit, without LDS or block barriers.
+// A round takes the wave's maximum over the experts still selectable (a NaN
+// never is), and the lowest id that holds it from one ballot per register.
+// Lane r then owns round r's selection; weights use topk_token's formulas and
+// summation orders, carried out identically in every lane.
+template <uint32_t R>
+__device__ void topk_token_wave(const uint16_t* lg, const void* bias, uint32_t* routes, uint32_t* telemetry,
+                                uint32_t b, const TopkParams& P, bool tel_is_lds) {
+    const uint32_t lane = threadIdx.x & 63, E = P.E, k = P.k;
+    float raw[R], s[R];
+    bool have[R];
+#pragma unroll
+    for (uint32_t i = 0; i < R; i++) {
+        const uint32_t e = lane + 64 * i;
+        have[i] = e < E;
+        float v = bf16_to_f32(lg[have[i] ? e : 0]);
+        if (P.mode == 0 && P.softcap > 0.0f) v = tanhf(v / P.softcap) * P.softcap;
+        raw[i] = v;
+    }
+    if (P.mode == 1) {
+        // initialize_softmax + activate_router_value, as in topk_token
+        float m = -INFINITY, den = 0.0f;
+        if (P.activation == 1) {
+#pragma unroll
+            for (uint32_t i = 0; i < R; i++)
+                if (have[i]) m = fmaxf(m, raw[i]);
+            for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
+#pragma unroll
+            for (uint32_t i = 0; i < R; i++)
+                if (have[i]) den += expf(raw[i] - m);
+            for (int d = 32; d > 0; d >>= 1) den += __shfl_xor(den, d);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < R; i++) {
+            float v = raw[i];
+            if (P.activation == 0) v = sigmoidf_(v);
+            else if (P.activation == 1) v = expf(v - m) / den;
+            else v = sqrtf(fmaxf(v, 0.0f) + logf(1.0f + expf(-fabsf(v))));
+            raw[i] = v;
+        }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < R; i++) {
+        const uint32_t e = have[i] ? lane + 64 * i : 0u;
+        s[i] = (P.mode == 0 && P.activation) ? sigmoidf_(raw[i]) : raw[i];
+        if (P.bias == 1) s[i] = s[i] + static_cast<const float*>(bias)[e];
+        else if (P.bias == 2) s[i] = s[i] + bf16_to_f32(static_cast<const uint16_t*>(bias)[e]);
+        have[i] = have[i] && s[i] == s[i];          // selectable: not a NaN, not yet taken
+    }
+    // Value of expert e (wave-uniform) in x.
+    auto value_of = [&](const float (&x)[R], uint32_t e) -> float {
+        float v = x[0];
+#pragma unroll
+        for (uint32_t i = 1; i < R; i++)
+            if (e >= 64 * i) v = x[i];
+        return lane_bcast(v, e & 63u);
+    };
+    uint32_t my_ex = 0;
+    float my_raw = 0.0f;
+    for (uint32_t r = 0; r < k; r++) {
+        float m = -INFINITY;
+#pragma unroll
+        for (uint32_t i = 0; i < R; i++)
+            if (have[i]) m = fmaxf(m, s[i]);
+        m = wave_max64(m);
+        uint32_t ex = 0xffffffffu;
+#pragma unroll
+        for (uint32_t i = 0; i < R; i++) {
+            const uint64_t at = __ballot(have[i] && s[i] == m);
+            if (ex == 0xffffffffu && at) ex = 64 * i + (uint32_t)__builtin_ctzll(at);
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < R; i++)
+            if (ex == lane + 64 * i) have[i] = false;
+        if (ex == 0xffffffffu) ex = 0;              // no selectable expert left
+        const float v = value_of(raw, ex);
+        if (lane == r) {
+            my_ex = ex;
+            my_raw = v;
+        }
+    }
+    const uint32_t total_sel = k + (P.mode == 1 ? P.always_count : 0u), total_res = E + (P.mode == 1 ? P.always_count : 0u);
+    float w;
+    if (P.mode == 0) {
+        const bool sig = P.activation != 0;
+        float maximum = lane_bcast(my_raw, 0), den = 0.0f;
+        if (P.normalize) {
+            const float term = sig ? sigmoidf_(my_raw) : expf(my_raw - maximum);
+            for (uint32_t r = 0; r < k; r++) den += lane_bcast(term, r);
+        } else if (!sig) {
+            maximum = -INFINITY;
+            for (uint32_t e = 0; e < E; e++) maximum = fmaxf(maximum, value_of(raw, e));
+            float term[R];
+#pragma unroll
+            for (uint32_t i = 0; i < R; i++) term[i] = expf(raw[i] - maximum);
+            for (uint32_t e = 0; e < E; e++) den += value_of(term, e);
+        }
+        w = sig ? sigmoidf_(my_raw) : expf(my_raw - maximum);
+        if (P.normalize || !sig) w /= den;
+    } else {
+        float den = 0.0f;
+        if (P.normalize)
+            for (uint32_t r = 0; r < k; r++) den += lane_bcast(my_raw, r);
+        w = P.normalize ? my_raw / den * P.routed_scale : my_raw * P.routed_scale;
+        if (lane >= k && lane < total_sel) {
+            my_ex = E + lane - k;
+            w = P.always_weight;
+        }
+    }
+    // Position in ascending expert order, equal ones in selection order (the
+    // reference's insertion sort); each pair of distinct experts counted once.
+    auto count = [&](uint32_t i) {
+        if (tel_is_lds) lds_count(&telemetry[i]);
+        else global_count(&telemetry[i]);
+    };
+    const bool mine = lane < total_sel;
+    uint32_t pos = 0;
+    for (uint32_t r = 0; r < total_sel; r++) {
+        const uint32_t ex = (uint32_t)__builtin_amdgcn_readlane((int)my_ex, (int)r);
+        pos += (ex < my_ex || (ex == my_ex && r < lane)) ? 1u : 0u;
+        if (telemetry && mine && r < lane && ex != my_ex) {
+            const uint32_t left = min(ex, my_ex), right = max(ex, my_ex);
+            count(total_res + left * (2u * total_res - left - 1u) / 2u + right - left - 1u);
+        }
+    }
+    if (!mine) return;
+    routes[(uint64_t)b * total_sel + pos] = (f32_to_bf16(w) << 16) | my_ex;
+    if (telemetry) count(my_ex);
+}
+
+// One wave's top-k for E <= 256 (total selections <= 64): the ranking form for
+// moe_topk with E <= 64, else the register rounds.  s_sh: the wave's LDS
+// scratch of 64 floats.
+__device__ __forceinline__ void topk_wave(const uint16_t* lg, const void* bias, uint32_t* routes, uint32_t* telemetry,
+                                          uint32_t b, const TopkParams& P, bool tel_is_lds, float* s_sh) {
+    if (P.E <= 64) {
+        if (P.mode == 0) topk_token_fast(lg, bias, routes, telemetry, b, true, P, tel_is_lds ? telemetry : nullptr, s_sh);
+        else topk_token_wave<1>(lg, bias, routes, telemetry, b, P, tel_is_lds);
+    } else if (P.E <= 128) {
+        topk_token_wave<2>(lg, bias, routes, telemetry, b, P, tel_is_lds);
+    } else {
+        topk_token_wave<4>(lg, bias, routes, telemetry, b, P, tel_is_lds);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // a7: route compaction (moe_route_compact_batch1.comp.template:26-106,
 // moe_route_count_batch1.comp.template:21-58) in one 1024-thread block.
@@ -665,7 +824,9 @@ __device__ void compact_body(const CompactArgs& A, uint32_t* scratch, uint32_t* 
         }
         return;
     }
-    if (A.n > blockDim.x && A.E <= COUNT_MAX_EXPERTS) {
+    // The counting sort from 65 routes on (600 routes: 5.6 us a launch against
+    // 35.4 for the rank loop, whose reads grow with n per route).
+    if (A.E <= COUNT_MAX_EXPERTS) {
         if (compact_counting(A, scratch, wave_tot, &misc[1])) return;
         __syncthreads();
     }
