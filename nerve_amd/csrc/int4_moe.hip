@@ -269,8 +269,277 @@ __global__ __launch_bounds__(64 * SM_WAVES) void sparse_int4_kernel(SmArgs A) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// Tiles of routes on the matrix cores (groups of whole 32-column blocks,
+// K % 128 == 0).
+//
+// A block owns a window of `group` route positions and 16 NW output channels.
+// Positions of one expert that follow each other in the map form a run (the
+// compaction sorts the map, so an expert is one run; an owned range leaves the
+// map in source order and the runs are shorter), and every TS-th position of a
+// run starts a tile of up to TS routes.  The block takes the tiles that start
+// in its window, so an expert's weights are decoded once per TS routes and not
+// once per route.
+//
+// A wave owns 16 channels: 16 weight rows of gate and the same of up (down: 32
+// rows).  Panels of PANEL columns of these rows stream through registers two
+// panels ahead (whole 128-byte lines, nontemporal: every block reads weights of
+// its own) into a wave-private LDS slot and are read back as MFMA operands: lane
+// (g = l / 16, r = l % 16) takes word g of a 32-column block of row r, which
+// the and-or expansion turns into the bf16 values 128 + q.  The tile's rows sit
+// in LDS in the pair order of that expansion.  Per block
+//   sum_k x (q - 8) = sum_k x (-136) + sum_k x (128 + q),
+// two chained MFMAs (the first one serves both row tiles; the matrix cores have
+// room for it, the LDS has little for stored sums), then acc = fma(that, scale,
+// acc).  Rows past the tile's count are never written: they only reach result
+// rows that are not stored.
+//
+// Bound: the weight stream (bytes of the distinct experts), with code expansion
+// and LDS reads each at about half of their units and a chain of five dependent
+// loads before a block's first weights.  Small panels and blocks (4 waves, 256
+// columns: three blocks a CU) hide that chain best: the routed block at h3072
+// i1024 e256 k10 with 16 tokens takes 180 us (213 with 512-column panels, 236
+// with a block per route), 64 tokens 396 (761), 256 tokens 594 (2673).
+// ---------------------------------------------------------------------------
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ uint32_t sm_pair_exponent() {   // see pair_exponent() of the INT4 linears
+    uint32_t e;
+    asm("v_mov_b32 %0, 0x43004300" : "=v"(e));
+    return e;
+}
+
+// LDS rows are padded by 16 bytes: 16 rows' operand reads hit distinct banks
+// at immediate offsets.  LDS bytes of one block:
+constexpr uint32_t tile_lds(uint32_t K, uint32_t TS, uint32_t NW, uint32_t PANEL) {
+    return TS * (K * 2 + 16) + NW * 2 * 16 * (PANEL / 2 + 16 + PANEL / 16);
+}
+
+template <bool GATE_UP, uint32_t TS, uint32_t NW, uint32_t PANEL, uint32_t WPE, bool SBF16>
+__global__ __launch_bounds__(64 * NW, WPE) void sparse_tile_kernel(SmArgs A, uint32_t group, uint32_t gshift) {
+    constexpr uint32_t PB = PANEL / 2, PP = PB / 16, PS = PANEL / 32;   // bytes, 16-byte pieces and scales of a panel row
+    constexpr uint32_t NL = 16 * PP / 64;                               // weight loads per lane, row tile and panel
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    __shared__ uint32_t t_route[TS], t_word[TS];
+    __shared__ uint32_t t_count;
+    const uint32_t K = A.K, N = A.N, ng = K / A.G, nblk = K / 32;   // G = 32 << gshift
+    const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const uint32_t g = lane >> 4, rr = lane & 15;
+    constexpr uint32_t WS = PB + 16;                                    // LDS stride of a weight row
+    const uint32_t xstr = K * 2 + 16;
+    uint8_t* xs = lds;                                                  // [TS] rows of K bf16 in pair order
+    uint8_t* slot = lds + TS * xstr + wave * (2 * 16 * (WS + 2 * PS));
+    uint16_t* sslot = reinterpret_cast<uint16_t*>(slot + 2 * 16 * WS);  // [2][16][PS]
+
+    const uint32_t w = (blockIdx.x % 8) * A.per_xcd + blockIdx.x / 8;
+    const uint32_t win = w % A.npos, tile = w / A.npos;                 // npos: windows
+    if (tile >= A.tiles) return;
+    const uint32_t cap = A.batch_width * A.k;
+    const uint32_t n0 = tile * (NW * 16 * (GATE_UP ? 1 : 2)) + wave * (GATE_UP ? 16 : 32);
+    const uint32_t exponent = sm_pair_exponent();
+
+    uint32_t start = 0, count = 0, npos = cap;
+    if (A.control) {
+        start = A.control[1];
+        count = A.control[2];
+        if (A.batched && count != 0u) npos = min(cap, A.control[3]);
+    }
+    // Route and expert of position p (0xffffffff: none).
+    auto route_at = [&](uint32_t p, uint32_t& c, uint32_t& word) -> uint32_t {
+        c = p;
+        word = 0;
+        if (p >= npos) return 0xffffffffu;
+        if (A.batched) c = A.frames[(uint64_t)(p / A.k) * A.frame_words + A.data_words + p % A.k];
+        if (c >= cap) return 0xffffffffu;
+        word = A.routes[c];
+        const uint32_t e = word & 0xffffu;
+        return (e >= A.E || (count != 0u && (e < start || e - start >= count))) ? 0xffffffffu : e;
+    };
+    for (uint32_t p = win * group; p < min(npos, (win + 1) * group); p++) {
+        // ---- the tile at position p, by every wave for itself: lane l looks
+        // at position p + l (the tile's routes) and p - 1 - l (the run's start).
+        uint32_t c, word, cb, wb;
+        const uint32_t ef = route_at(p + lane, c, word);
+        uint32_t eb = route_at(lane < p ? p - 1 - lane : 0xffffffffu, cb, wb);
+        const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)ef);
+        if (e == 0xffffffffu) continue;
+        uint32_t back = 0;                                              // positions of the run before p
+        for (;;) {
+            const uint64_t other = __ballot(eb != e);
+            if (other) {
+                back += (uint32_t)__builtin_ctzll(other);
+                break;
+            }
+            back += 64;
+            eb = route_at(back + lane < p ? p - 1 - back - lane : 0xffffffffu, cb, wb);
+        }
+        if (back % TS) continue;
+        const uint64_t fend = __ballot(ef != e);
+        const uint32_t nt = min(TS, fend ? (uint32_t)__builtin_ctzll(fend) : 64u);
+        const uint32_t* W = static_cast<const uint32_t*>(sm_param(A, 2 * e, A.w_bytes, 16));
+        const uint16_t* S = static_cast<const uint16_t*>(sm_param(A, 2 * e + 1, A.s_bytes, 2));
+        if (!W || !S) continue;                                         // uniform over the block
+        __syncthreads();                                                // the previous tile's reads are done
+        if (tid < TS) {
+            t_route[tid] = c;
+            t_word[tid] = word;
+        }
+        // ---- weight stream: row tile m's 16 rows start at row0[m].
+        const uint32_t row0[2] = {min(n0, N - 16), GATE_UP ? A.I + min(n0, N - 16) : min(n0 + 16, N - 16)};
+        const bool words = gshift == 0 && ((uintptr_t)S & 3) == 0;          // scales in dwords (K / 32 is even)
+        struct Panel {
+            v4i w[2][NL];
+            uint32_t s[2][PS / 8];
+        };
+        auto load = [&](Panel& R, uint32_t k0) __attribute__((always_inline)) {
+            if (k0 >= K) return;
+#pragma unroll
+            for (uint32_t m = 0; m < 2; m++) {
+#pragma unroll
+                for (uint32_t i = 0; i < NL; i++) {
+                    const uint32_t x = i * 64 + lane, row = x / PP, pc = x % PP;
+                    const v4i* wp = reinterpret_cast<const v4i*>(W + (uint64_t)(row0[m] + row) * (K / 8) + min(k0 / 32 + pc, nblk - 1) * 4);
+                    R.w[m][i] = TS < 16 ? __builtin_nontemporal_load(wp) : *wp;
+                }
+                // Scales: lane (g, r) loads blocks PS / 4 g .. of row r.
+                const uint16_t* sp = S + (uint64_t)(row0[m] + rr) * ng;
+#pragma unroll
+                for (uint32_t i = 0; i < PS / 8; i++) {
+                    const uint32_t b = min(k0 / 32 + PS / 4 * g + 2 * i, nblk - 2);
+                    if (words) R.s[m][i] = *reinterpret_cast<const uint32_t*>(sp + b);
+                    else R.s[m][i] = (uint32_t)sp[b >> gshift] | ((uint32_t)sp[(b + 1) >> gshift] << 16);
+                }
+            }
+        };
+        Panel ra, rb;
+        load(ra, 0);
+        load(rb, PANEL);
+        __syncthreads();                                                // t_route is written
+        // ---- the tile's rows into LDS
+        for (uint32_t x = tid; x < nt * (K / 8); x += 64 * NW) {
+            const uint32_t t = x / (K / 8), o = x % (K / 8);
+            const uint32_t ct = t_route[t], b = ct / A.k, r = ct % A.k;
+            const uint16_t* xg = GATE_UP ? A.x + (uint64_t)b * K : A.x + (uint64_t)b * A.frame_words * 2 + (uint64_t)r * A.I;
+            v4i v;
+            __builtin_memcpy(&v, __builtin_assume_aligned(xg + 8 * o, 4), 16);
+            *reinterpret_cast<v4i*>(xs + t * xstr + o * 16) = sm_permute(v);
+        }
+        __syncthreads();
+        v4f acc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+        const v4i minus136 = v4i{(int)0xC308C308u, (int)0xC308C308u, (int)0xC308C308u, (int)0xC308C308u};
+        const uint32_t tr = rr % TS;
+        auto contract = [&](Panel& R, uint32_t k0) __attribute__((always_inline)) {
+#pragma unroll
+            for (uint32_t m = 0; m < 2; m++) {
+#pragma unroll
+                for (uint32_t i = 0; i < NL; i++) {
+                    const uint32_t x = i * 64 + lane, row = x / PP, pc = x % PP;
+                    *reinterpret_cast<v4i*>(slot + (m * 16 + row) * WS + pc * 16) = R.w[m][i];
+                }
+#pragma unroll
+                for (uint32_t i = 0; i < PS / 8; i++)
+                    *reinterpret_cast<uint32_t*>(sslot + (m * 16 + rr) * PS + PS / 4 * g + 2 * i) = R.s[m][i];
+            }
+            load(R, k0 + 2 * PANEL);
+            __builtin_amdgcn_wave_barrier();
+            const uint8_t* xp = xs + tr * xstr + k0 * 2 + 16 * g;
+            const uint8_t* wq = slot + rr * WS + 4 * g;
+#pragma unroll
+            for (uint32_t ch = 0; ch < PANEL / 128; ch++) {
+                if (k0 + 128 * ch >= K) break;                          // uniform
+                v2i sv[2];
+#pragma unroll
+                for (uint32_t m = 0; m < 2; m++) sv[m] = *reinterpret_cast<const v2i*>(sslot + (m * 16 + rr) * PS + 4 * ch);
+#pragma unroll
+                for (uint32_t u = 0; u < 4; u++) {
+                    const uint32_t pc = 4 * ch + u;
+                    const v4i av = *reinterpret_cast<const v4i*>(xp + pc * 64);
+                    const v4f cs = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, av), __builtin_bit_cast(v8bf, minus136),
+                                                                           v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+                    for (uint32_t m = 0; m < 2; m++) {
+                        const uint32_t wd = *reinterpret_cast<const uint32_t*>(wq + m * 16 * WS + pc * 16);
+                        const v4i bw = v4i{(int)((wd & 0x000F000Fu) | exponent), (int)(((wd >> 4) & 0x000F000Fu) | exponent),
+                                           (int)(((wd >> 8) & 0x000F000Fu) | exponent), (int)(((wd >> 12) & 0x000F000Fu) | exponent)};
+                        const v4f d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, av),
+                                                                              __builtin_bit_cast(v8bf, bw), cs, 0, 0, 0);
+                        const uint32_t sb = (uint32_t)sv[m][u / 2];
+                        const float sc = !SBF16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)(u % 2 ? sb >> 16 : sb))
+                                         : __uint_as_float(u % 2 ? sb & 0xffff0000u : sb << 16);
+#pragma unroll
+                        for (int i = 0; i < 4; i++) acc[m][i] = fmaf(d[i], sc, acc[m][i]);
+                    }
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        };
+        for (uint32_t k0 = 0; k0 < K; k0 += 2 * PANEL) {
+            contract(ra, k0);
+            if (k0 + PANEL < K) contract(rb, k0 + PANEL);
+        }
+        // ---- result lane (g, r): routes 4 g + i, row r of each row tile.
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            const uint32_t t = 4 * g + i;
+            if (t >= nt) continue;
+            const uint32_t ct = t_route[t % TS];
+            if constexpr (GATE_UP) {
+                // …gate_up_int4_ct.comp.template:205-213
+                if (n0 + rr >= N) continue;
+                const float gv = round_bf16(acc[0][i]), uv = round_bf16(acc[1][i]);
+                const float act = round_bf16(round_bf16(gv / (1.0f + expf(-gv))) * uv);
+                A.out[(uint64_t)(ct / A.k) * A.frame_words * 2 + (uint64_t)(ct % A.k) * A.I + n0 + rr] = (uint16_t)f32_to_bf16(act);
+            } else {
+                // …down_int4_ct.comp.template:176-181
+                const float wr = bf16_to_f32(t_word[t % TS] >> 16);
+#pragma unroll
+                for (uint32_t m = 0; m < 2; m++)
+                    if (n0 + 16 * m + rr < N)
+                        A.out[(uint64_t)ct * N + n0 + 16 * m + rr] = (uint16_t)f32_to_bf16(round_bf16(round_bf16(acc[m][i]) * wr));
+            }
+        }
+    }
+}
+
+template <bool GATE_UP, uint32_t TS, uint32_t NW, uint32_t PANEL, uint32_t WPE>
+nerve_hip_status launch_tile_form(SmArgs A, uint32_t group, hipStream_t stream) {
+    const uint32_t rows = NW * 16 * (GATE_UP ? 1 : 2), lds = tile_lds(A.K, TS, NW, PANEL);
+    A.tiles = (A.N + rows - 1) / rows;
+    A.npos = (A.npos + group - 1) / group;
+    A.per_xcd = (uint32_t)(((uint64_t)A.npos * A.tiles + 7) / 8);
+    auto* kernel = A.scale_bf16 ? sparse_tile_kernel<GATE_UP, TS, NW, PANEL, WPE, true> : sparse_tile_kernel<GATE_UP, TS, NW, PANEL, WPE, false>;
+    static bool attr_set[2] = {false, false};
+    if (!attr_set[A.scale_bf16 ? 1 : 0]) {
+        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256) != hipSuccess)
+            return nh::fail(NERVE_HIP_DEVICE_ERROR, "hipFuncSetAttribute failed for sparse_tile_kernel");
+        attr_set[A.scale_bf16 ? 1 : 0] = true;
+    }
+    kernel<<<A.per_xcd * 8, 64 * NW, lds, stream>>>(A, group, (uint32_t)__builtin_ctz(A.G / 32));
+    return nh::check_launch(GATE_UP ? "int4_moe_gate_up" : "int4_moe_down");
+}
+
+// The tile form, or UNSUPPORTED where its loads or its LDS do not fit.
+template <bool GATE_UP>
+nerve_hip_status launch_tiles(const SmArgs& A, hipStream_t stream) {
+    constexpr uint32_t MOST = 160 * 1024 - 256;
+    if (A.G % 32 || (A.G & (A.G - 1)) || A.K % 128 || A.N % 16) return NERVE_HIP_UNSUPPORTED;
+    // Routes per expert if they spread evenly: a tile takes 4, 8 or 16 routes,
+    // since its rows in LDS (2 K bytes each) cost blocks per CU.  The routed
+    // block at h3072 i1024 e256 k10, us by tile size 4 / 8 / 16 at 16, 64 and
+    // 256 tokens: 180 / 191 / 219, 396 / 403 / 457, 976 / 740 / 594.  Windows of
+    // 8 positions where most of them start no tile.
+    const uint32_t per = A.npos / A.E;
+    const uint32_t group = per >= 4 ? 8 : 1;
+    if (per < 3 && tile_lds(A.K, 4, 4, 256) <= MOST) return launch_tile_form<GATE_UP, 4, 4, 256, 3>(A, group, stream);
+    if (per < 8 && tile_lds(A.K, 8, 4, 256) <= MOST) return launch_tile_form<GATE_UP, 8, 4, 256, 2>(A, group, stream);
+    if (tile_lds(A.K, 16, 8, 256) <= MOST) return launch_tile_form<GATE_UP, 16, 8, 256, 2>(A, group, stream);
+    return NERVE_HIP_UNSUPPORTED;
+}
+
 template <bool GATE_UP>
 nerve_hip_status launch_sparse(const SmArgs& A, hipStream_t stream) {
+    const nerve_hip_status tiled = launch_tiles<GATE_UP>(A, stream);
+    if (tiled != NERVE_HIP_UNSUPPORTED) return tiled;
     const uint32_t units = A.K / 32;
     const bool spw = A.G % 32 != 0;
     const uint32_t lu = units % 64 == 0 ? 64u : (units % 32 == 0 || units > 32) ? 32u : 16u;

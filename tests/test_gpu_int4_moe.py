@@ -140,6 +140,30 @@ def test_batched_shapes(ctx, dev, H, I, G, sbf, B):
     _check(rig, x, routes, h, y)
 
 
+# The matrix-core tile form: every tile size (4, 8, 16 routes, by routes per
+# expert), runs cut at a tile and longer than a wave (the run's start is then
+# searched over several rounds), windows of one and eight positions, one panel,
+# a panel and a half and an odd number of them, output rows cut at a block's
+# channels, f16 and bf16 scales of one and several blocks, and an owned range
+# (runs of a map in source order).
+@pytest.mark.parametrize("H,I,G,sbf,E,k,B,owned", [
+    (128, 128, 32, True, 8, 2, 5, None),
+    (384, 640, 32, False, 16, 3, 20, None),
+    (640, 128, 64, True, 4, 2, 9, None),
+    (256, 384, 128, False, 3, 2, 70, None),
+    (512, 256, 32, True, 2, 1, 300, None),
+    (384, 128, 32, True, 6, 3, 50, (2, 3)),
+])
+def test_tile_form(ctx, dev, H, I, G, sbf, E, k, B, owned):
+    rig = Rig(dev, H, I, E, k, G, sbf, nb=E, seed=H + I + B)
+    routes, _ = oracle.topk(wl.bf16_normal(rig.rng, (B, E)), k, telemetry=False)
+    routes = routes.astype(np.uint32)
+    x = wl.bf16_normal(rig.rng, (B, H))
+    start, count = owned or (0, 0)
+    h, y, _, _ = _run_batched(ctx, rig, x, routes, B, start, count)
+    _check(rig, x, routes, h, y, start, count)
+
+
 @pytest.mark.parametrize("start,count", [(4, 6), (0, 1), (15, 1)])
 def test_owned_expert_range(ctx, dev, start, count):
     E, k, B, H, I, G = 16, 4, 6, 512, 256, 32
