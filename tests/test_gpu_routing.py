@@ -99,6 +99,40 @@ def test_topk_routed(ctx, dev, B, E, k, sigmoid, normalize, softcap, bias):
     assert np.array_equal(to_np(tel, np.uint32), ref_tel)  # telemetry counts exact
 
 
+# The register rounds at two and four experts a lane, the block's telemetry
+# counts in LDS (256 tokens on; 176 experts' counters no longer fit) and a last
+# block with idle waves.
+@pytest.mark.parametrize("B,E,k,sigmoid,normalize,mode", [
+    (3, 65, 5, False, False, 0), (257, 128, 8, False, True, 0), (300, 64, 6, True, True, 0),
+    (260, 256, 10, False, False, 0), (270, 174, 7, True, False, 0), (258, 100, 4, False, True, 1),
+    (5, 200, 60, False, True, 1)])
+def test_topk_wave_forms(ctx, dev, B, E, k, sigmoid, normalize, mode):
+    torch = _torch()
+    rng = np.random.default_rng(B + E + k)
+    logits = wl.bf16_normal(rng, (B, E), 2.0)
+    logits[1, E - 1] = logits[1, 1] = logits[1, 64 % E] = wl.f32_to_bf16_bits(np.float32(9.0))   # ties
+    logits[2, E // 2] = 0x7FC0                                                                    # a NaN
+    A = 3 if mode else 0
+    bias = rng.standard_normal(E).astype(np.float32) * np.float32(0.01) if mode else None
+    spec = (f"moe_router_batch1_score_topk_softmax_bf16_r{E}_k{k}_a{A}w0.5_norm1_scale2.5_biasf32.comp" if mode
+            else topk_spec(E, k, sigmoid=sigmoid, normalize=normalize))
+    if mode:
+        logits[2, E // 2] = 0x3F80          # a NaN would spread over the whole softmax
+    T = E + A
+    routes = torch.zeros(B, k + A, dtype=torch.int32, device=dev)
+    tel = torch.zeros(T + T * (T - 1) // 2, dtype=torch.int32, device=dev)
+    ctx.moe_router_topk(spec, to_dev(logits, dev), None if bias is None else to_dev(bias, dev), routes, tel, B)
+    ref, ref_tel = oracle.topk(logits, k, mode=mode, activation=1 if mode else int(sigmoid), normalize=int(normalize),
+                               **(dict(routed_scale=2.5, always_count=A, always_weight=0.5, bias=bias) if mode else {}))
+    gi, gw = _route_split(to_np(routes, np.uint32))
+    ri, rw = _route_split(ref)
+    assert np.array_equal(gi, ri)
+    finite = np.isfinite(rw)          # a full softmax over a row with a NaN has NaN weights on both sides
+    assert np.array_equal(finite, np.isfinite(gw))
+    assert np.allclose(gw[finite], rw[finite], rtol=2e-2, atol=1e-6)
+    assert np.array_equal(to_np(tel, np.uint32), ref_tel)
+
+
 @pytest.mark.parametrize("act", ["sigmoid", "softmax", "sqrtsoftplus"])
 def test_score_router(ctx, dev, act):
     torch = _torch()
@@ -121,8 +155,8 @@ def test_score_router(ctx, dev, act):
 
 
 # n = B k routes: one wave's ballot ranks (n <= 64), the counting sort with
-# each wave's segment in registers (1024 < n <= 8192; 8192 fills them), its
-# looped form (n > 8192), and the rank loop (64 < n <= 1024).
+# each wave's segment in registers (64 < n <= 8192; 8192 fills them) and its
+# looped form (n > 8192).
 @pytest.mark.parametrize("B,k,E", [(16, 4, 32), (2048, 4, 128), (1, 1, 8), (300, 6, 64), (2100, 4, 128),
                                    (100, 4, 32)])
 @pytest.mark.parametrize("partition", [None, (8, 20)])
