@@ -156,7 +156,9 @@ def _stream(stream) -> int | None:
     if stream is None:
         import torch
 
-        return torch.cuda.current_stream().cuda_stream
+        # The current stream's handle without building a Stream object: 0.3 us
+        # of a 6.9 us call instead of 2.8.
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     return stream if isinstance(stream, int) else stream.cuda_stream
 
 
