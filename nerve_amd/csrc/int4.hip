@@ -15,6 +15,8 @@
 // A row r and of B column r for its k-slice; both operands are loaded in the
 // same per-lane k order, so A/B pairing is the identity.  Result lane (g, r)
 // holds D[4g+i][r].
+#include <algorithm>
+
 #include "int4_dev.h"
 
 namespace {
@@ -238,7 +240,7 @@ __device__ __forceinline__ float sum8_bf16(v4i v) {
 }
 
 template <int KS, int G, bool ZP, uint32_t MT>
-__global__ __launch_bounds__(64 * KS) void int4_gptq_gemv_kernel(Int4Args A) {
+__global__ __launch_bounds__(64 * KS) void int4_gptq_gemv_kernel(Int4Args A, float* split_part) {
     constexpr uint32_t GR = G / 8;                 // packed rows per group
     constexpr uint32_t GPB = GEMV_ROWS / GR;       // groups per batch
     constexpr uint32_t LR = GEMV_ROWS / 4;         // packed rows per lane per batch
@@ -255,9 +257,11 @@ __global__ __launch_bounds__(64 * KS) void int4_gptq_gemv_kernel(Int4Args A) {
     if (n0 >= N) return;
     const uint32_t col = n0 + 4 * c;               // first of the lane's 4 columns
     const uint32_t ngroups = K / G;
-    const uint32_t nbatch = (ngroups + GPB - 1) / GPB;
-    const uint32_t per = (nbatch + KS - 1) / KS;
-    const uint32_t b0 = min(nbatch, wave * per), b1 = min(nbatch, b0 + per);
+    // This split's batches of K (gridDim.y splits), dealt to the waves.
+    const uint32_t batches = (ngroups + GPB - 1) / GPB;
+    const uint32_t s0 = batches * blockIdx.y / gridDim.y, nbatch = batches * (blockIdx.y + 1) / gridDim.y;
+    const uint32_t per = (nbatch - s0 + KS - 1) / KS;
+    const uint32_t b0 = min(nbatch, s0 + wave * per), b1 = min(nbatch, b0 + per);
     const uint32_t zshift = 4 * (col % 8);
     v4f acc[MT];
 #pragma unroll
@@ -336,74 +340,119 @@ __global__ __launch_bounds__(64 * KS) void int4_gptq_gemv_kernel(Int4Args A) {
         float v = pf[t * 64 + lane];
 #pragma unroll
         for (int w2 = 1; w2 < KS; w2++) v += pf[(w2 * MT + t) * 64 + lane];
-        finalize_store(A, t, n0 + lane, v);
+        if (split_part) split_part[((uint64_t)blockIdx.y * M + t) * N + n0 + lane] = v;
+        else finalize_store(A, t, n0 + lane, v);
     }
 }
 
-// CT layout: qweight [N, K/8], scales [N, K/G], G % 128 == 0.  A wave owns 16
-// columns; per 128-k step lane (g, r) loads 4 consecutive words of column r
-// (k-slices 4g..4g+3) and MFMA j contracts slice 4g+j of every lane group.
-template <int KS>
-__global__ __launch_bounds__(64 * KS) void int4_ct_kernel(Int4Args A) {
-    __shared__ v4f part[KS][64];
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+// CT layout: qweight [N, K/8], scales [N, K/G], G % 128 == 0.  A block owns 16 J
+// rows of weights (output columns) and 16 tokens; its KS waves split the 128-k
+// steps of K in batches of four (512 columns).  A batch's weights are read 256
+// contiguous bytes per row (lane l: 16-byte piece l % 16 of rows l / 16 + 4 i),
+// nontemporal when one token tile reads them, pass through a wave-private LDS
+// slot (rows padded by 16 bytes: operand reads of 16 rows hit distinct banks)
+// and come back as lane (g, r)'s 4 consecutive words of row r (k-slices 4g..4g+3
+// of a step); MFMA j contracts slice 4g+j of every lane group.
+//
+// Bound: the weight stream; from about 8 tokens on the activation rows each
+// block re-reads (J = 2 halves them).  One register set and 16 waves a CU
+// (<= 128 registers) stream better than two sets and 8: 4096 x 14336, one token
+// 12.6 us against 15.5; 16.1 when the weights were read in the operand layout
+// (64 bytes per row and instruction) and the scales at the fold.  J = 2 needs 144
+// registers (held to 128 it spills: 16 tokens 21.0 us against 17.7; 25.6 before).
+// 14336 x 4096, one token: 17.1 -> 11.5.
+constexpr uint32_t CT_BATCH = 4;
+constexpr uint32_t CT_STRIDE = CT_BATCH * 64 + 16;
+
+template <int KS, int J>
+__global__ __launch_bounds__(64 * KS, J == 1 ? 4 : 2) void int4_ct_kernel(Int4Args A) {
+    __shared__ __attribute__((aligned(16))) uint8_t slots[KS][J * 16 * CT_STRIDE];   // then the wave's partial sums
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const uint32_t g = lane >> 4, rr = lane & 15;
-    const uint32_t n = blockIdx.x * 16 + rr;
-    const uint32_t m0 = blockIdx.y * 16;
+    const uint32_t n0 = blockIdx.x * 16 * J, m0 = blockIdx.y * 16;
     const uint32_t tok = m0 + rr;
-    const uint32_t ngroups = A.K / A.G, steps = A.G / 128;
-    const uint32_t per = (ngroups + KS - 1) / KS;
-    const uint32_t g0 = min(ngroups, wave * per), g1 = min(ngroups, g0 + per);
+    const uint32_t ngroups = A.K / A.G, steps = A.G / 128, nstep = A.K / 128;
+    const uint32_t per = (nstep + KS - 1) / KS;
+    const uint32_t first = min(nstep, wave * per), last = min(nstep, first + per);
     const bool tv = tok < A.B;
-    const uint16_t* xrow = A.x + (uint64_t)(tv ? tok : 0) * A.K;
-    const uint32_t* wrow = A.qw + (uint64_t)n * (A.K / 8);
-    v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
-    v4f ag = v4f{0.f, 0.f, 0.f, 0.f}, as = v4f{0.f, 0.f, 0.f, 0.f};
-    // 128-k steps run in batches of CT_BATCH with every load of a batch issued
-    // before its first MFMA; a group is scaled and folded into acc after its
-    // last step.
-    constexpr uint32_t CT_BATCH = 4;
-    const uint32_t first = g0 * steps, last = g1 * steps;
+    const uint16_t* xrow = A.x + (uint64_t)(tv ? tok : 0) * A.K + 32 * g;
+    const uint32_t* wrow = A.qw + (uint64_t)(n0 + g) * (A.K / 8);          // row l / 16 of the load pattern
+    const uint16_t* srow = A.scales + (uint64_t)(n0 + rr) * ngroups;
+    const uint32_t exponent = pair_exponent();
+    uint8_t* slot = slots[wave];
+    struct Batch {
+        v4i w[J][4], a[CT_BATCH][4];
+        uint16_t s[J][CT_BATCH];
+    };
+    auto load = [&](Batch& B, uint32_t base) __attribute__((always_inline)) {
+        const uint32_t pc = min(base * 4 + rr, last * 4 - 1);
+#pragma unroll
+        for (int j = 0; j < J; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const v4i* p = reinterpret_cast<const v4i*>(wrow + (uint64_t)(16 * j + 4 * i) * (A.K / 8) + pc * 4);
+                B.w[j][i] = gridDim.y == 1 ? __builtin_nontemporal_load(p) : *p;
+            }
+#pragma unroll
+        for (uint32_t u = 0; u < CT_BATCH; u++) {
+            const uint32_t i = min(base + u, last - 1);
+#pragma unroll
+            for (int j = 0; j < 4; j++) B.a[u][j] = tv ? *reinterpret_cast<const v4i*>(xrow + i * 128 + 8 * j) : v4i{0, 0, 0, 0};
+#pragma unroll
+            for (int j = 0; j < J; j++) B.s[j][u] = srow[(uint64_t)(16 * j) * ngroups + i / steps];
+        }
+    };
+    v4f acc[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+    const v4i ones = v4i{(int)ONES_BF16, (int)ONES_BF16, (int)ONES_BF16, (int)ONES_BF16};
+    auto contract = [&](Batch& B, uint32_t base) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < J; j++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                *reinterpret_cast<v4i*>(slot + (16 * j + 4 * i + g) * CT_STRIDE + rr * 16) = B.w[j][i];
+        __builtin_amdgcn_wave_barrier();
+        // A step's sums are folded by its own scale (a group's steps share one).
+#pragma unroll
+        for (uint32_t u = 0; u < CT_BATCH; u++) {
+            if (base + u >= last) break;
+            v4i ap[4];
+            v4f as = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                ap[q] = permute_act(B.a[u][q]);
+                as = mfma_bf16(ap[q], ones, as);
+            }
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                const v4i w = *reinterpret_cast<const v4i*>(slot + (16 * j + rr) * CT_STRIDE + (4 * u + g) * 16);
+                v4f ag = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int q = 0; q < 4; q++) ag = mfma_bf16(ap[q], dequant_word((uint32_t)w[q], exponent), ag);
+                const float sc = decode_scale(B.s[j][u], A.scale_bf16);
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[j][i] = fmaf(sc, ag[i] - 136.0f * as[i], acc[j][i]);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    Batch p;
     for (uint32_t base = first; base < last; base += CT_BATCH) {
-        v4i wbuf[CT_BATCH], abuf[CT_BATCH][4];
-#pragma unroll
-        for (uint32_t u = 0; u < CT_BATCH; u++) {
-            const uint32_t kb = min(base + u, last - 1) * 128;
-            wbuf[u] = *reinterpret_cast<const v4i*>(wrow + kb / 8 + 4 * g);
-            const uint16_t* xa = xrow + kb + 32 * g;
-#pragma unroll
-            for (int j = 0; j < 4; j++) abuf[u][j] = tv ? *reinterpret_cast<const v4i*>(xa + 8 * j) : v4i{0, 0, 0, 0};
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < CT_BATCH; u++) {
-            const uint32_t i = base + u;
-            if (i >= last) break;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                v4i ap = permute_act(abuf[u][j]);
-                uint32_t wj = (uint32_t)(j == 0 ? wbuf[u].x : j == 1 ? wbuf[u].y : j == 2 ? wbuf[u].z : wbuf[u].w);
-                ag = mfma_bf16(ap, dequant_word(wj), ag);
-                as = mfma_bf16(ap, v4i{(int)ONES_BF16, (int)ONES_BF16, (int)ONES_BF16, (int)ONES_BF16}, as);
-            }
-            if ((i + 1) % steps == 0) {
-                float sc = load_scale(A.scales + (uint64_t)n * ngroups + i / steps, A.scale_bf16);
-#pragma unroll
-                for (int q = 0; q < 4; q++) acc[q] = fmaf(sc, ag[q] - 136.0f * as[q], acc[q]);
-                ag = v4f{0.f, 0.f, 0.f, 0.f};
-                as = v4f{0.f, 0.f, 0.f, 0.f};
-            }
-        }
+        load(p, base);
+        contract(p, base);
     }
-    part[wave][lane] = acc;
-    __syncthreads();
-    if (wave != 0) return;
-    v4f t = part[0][lane];
 #pragma unroll
-    for (int w = 1; w < KS; w++) t += part[w][lane];
+    for (int j = 0; j < J; j++) reinterpret_cast<v4f*>(slot)[j * 64 + lane] = acc[j];
+    __syncthreads();
+    if (wave >= J) return;
+    v4f t = reinterpret_cast<const v4f*>(slots[0])[wave * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < KS; w++) t += reinterpret_cast<const v4f*>(slots[w])[wave * 64 + lane];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        uint32_t tt = m0 + 4 * g + i;
-        if (tt < A.B) finalize_store(A, tt, n, t[i]);
+        const uint32_t tt = m0 + 4 * g + i;
+        if (tt < A.B) finalize_store(A, tt, n0 + 16 * wave + rr, t[i]);
     }
 }
 
@@ -806,13 +855,16 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
     A.scale_bf16 = s.scale_bf16;
     A.finalize = s.op;
     hipStream_t strm = (hipStream_t)stream;
-    // More than 16 rows: the tiled split-K form, which expands the weights once
+    // Five rows on, few column tiles and a long K: also the split-K form (16 rows
+    // of 14336 x 4096: 25.4 -> 14.6 us).  More than 16 rows: the tiled split-K form, which expands the weights once
     // per 64 rows instead of once per 16.  The 16-row kernels stay where one
     // round of their blocks covers a GPTQ linear with a short K (64 rows of
     // 4096 x 4096: 10.1 against 15.1 us; of 14336 x 4096: 25.9 against 20.0).
     const bool one_round = s.layout == 0 && A.N % 64 == 0 && A.K <= 6144 &&
                            (uint64_t)(A.N / 64) * ((batch_width + 15) / 16) <= (uint64_t)ctx->cu_count;
-    if (batch_width > 16 && !one_round && !(s.layout == 1 && (zeros || A.G % 128)) &&
+    const bool few = s.layout == 0 && A.N % 64 == 0 && batch_width > GEMV_MAX_M && A.K > 6144 &&
+                     2 * (A.N / 64) <= (uint32_t)ctx->cu_count;
+    if (((batch_width > 16 && !one_round) || few) && !(s.layout == 1 && (zeros || A.G % 128)) &&
         nh::int4_gemm(ctx, A, nullptr, false, s.layout == 1, strm))
         return nh::check_launch("int4_linear_gemm");
     if (s.layout == 0) {
@@ -828,18 +880,24 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
         // Decode-sized batches go to the vector-ALU kernel.
         if (wide && batch_width <= GEMV_MAX_M && (A.G == 32 || A.G == 64 || A.G == 128 || A.G == 256) &&
             ((uintptr_t)scales & 7) == 0) {
-            dim3 g1((tiles + 7) / 8 * 8);
+            // Few column tiles and more than one batch per wave: K is split so
+            // that every CU has a block, the partial sums added by a second
+            // launch (14336 x 4096, one row: 64 blocks 14.9 us, 256 10.1).
+            const uint32_t splits = std::max(1u, std::min((A.K / 256 + 15) / 16, (uint32_t)ctx->cu_count / tiles));
+            float* part = splits > 1 ? static_cast<float*>(ctx->split) : nullptr;
+            dim3 g1((tiles + 7) / 8 * 8, splits);
             const bool zp = zeros != nullptr;
 #define NERVE_INT4_GEMV(GG)                                                                   \
-    (batch_width == 1 ? (zp ? int4_gptq_gemv_kernel<16, GG, true, 1><<<g1, 1024, 0, strm>>>(A)   \
-                            : int4_gptq_gemv_kernel<16, GG, false, 1><<<g1, 1024, 0, strm>>>(A)) \
-                      : (zp ? int4_gptq_gemv_kernel<16, GG, true, 4><<<g1, 1024, 0, strm>>>(A)   \
-                            : int4_gptq_gemv_kernel<16, GG, false, 4><<<g1, 1024, 0, strm>>>(A)))
+    (batch_width == 1 ? (zp ? int4_gptq_gemv_kernel<16, GG, true, 1><<<g1, 1024, 0, strm>>>(A, part)   \
+                            : int4_gptq_gemv_kernel<16, GG, false, 1><<<g1, 1024, 0, strm>>>(A, part)) \
+                      : (zp ? int4_gptq_gemv_kernel<16, GG, true, 4><<<g1, 1024, 0, strm>>>(A, part)   \
+                            : int4_gptq_gemv_kernel<16, GG, false, 4><<<g1, 1024, 0, strm>>>(A, part)))
             if (A.G == 128) NERVE_INT4_GEMV(128);
             else if (A.G == 64) NERVE_INT4_GEMV(64);
             else if (A.G == 32) NERVE_INT4_GEMV(32);
             else NERVE_INT4_GEMV(256);
 #undef NERVE_INT4_GEMV
+            if (part) nh::int4_split_sum(A, part, splits, strm);
             return nh::check_launch("int4_linear_gptq_gemv");
         }
         // Few column tiles (decode-sized N): 16 waves split K so that each
@@ -857,8 +915,13 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
     }
     if (zeros) return nh::fail(NERVE_HIP_UNSUPPORTED, "asymmetric zeros are supported for the GPTQ layout only");
     if (A.G % 128 || A.N % 16) return nh::fail(NERVE_HIP_UNSUPPORTED, "CT INT4 kernel needs group % 128 == 0 and N % 16 == 0");
-    dim3 grid(A.N / 16, (batch_width + 15) / 16);
-    int4_ct_kernel<8><<<grid, 512, 0, strm>>>(A);
+    // 32 rows a block where that still gives every CU one and the activations
+    // count (16 tokens of 4096 x 14336: 17.7 us against 22.0; one: 12.9, 12.6).
+    const uint32_t row_tiles = (batch_width + 15) / 16;
+    if (batch_width > 2 && A.N % 32 == 0 && A.N / 32 * row_tiles >= (uint32_t)ctx->cu_count)
+        int4_ct_kernel<8, 2><<<dim3(A.N / 32, row_tiles), 512, 0, strm>>>(A);
+    else
+        int4_ct_kernel<8, 1><<<dim3(A.N / 16, row_tiles), 512, 0, strm>>>(A);
     return nh::check_launch("int4_linear_ct");
 }
 

@@ -110,4 +110,7 @@ namespace nh {
 // `i8` is null for bf16 activations.
 bool int4_gemm(const nerve_hip_ctx* ctx, const Int4Args& A, const PpArgs* i8, bool paired, bool ct, hipStream_t st);
 
+// Adds the partial sums f32 [splits][B][N] in split order, finalizes and stores.
+void int4_split_sum(const Int4Args& A, const float* part, uint32_t splits, hipStream_t st);
+
 }  // namespace nh

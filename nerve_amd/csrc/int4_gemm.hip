@@ -351,19 +351,18 @@ __global__ __launch_bounds__(GT_THREADS, 2) void int4_gemm_kernel(GemmArgs P) {
 
 // Partial sums in split order, then bias or residual and the bf16 store: four
 // columns per thread, eight splits' loads in flight.
-__global__ __launch_bounds__(256) void int4_split_sum_kernel(GemmArgs P) {
-    const Int4Args& A = P.L;
+__global__ __launch_bounds__(256) void int4_split_sum_kernel(Int4Args A, const float* part, uint32_t splits) {
     const uint64_t i = ((uint64_t)blockIdx.x * 256 + threadIdx.x) * 4, total = (uint64_t)A.B * A.N;
     if (i >= total) return;
-    const float* p = P.part + i;
+    const float* p = part + i;
     v4f v = v4f{0.f, 0.f, 0.f, 0.f};
-    for (uint32_t s = 0; s < P.splits; s += 8) {
+    for (uint32_t s = 0; s < splits; s += 8) {
         v4f t[8];
 #pragma unroll
-        for (uint32_t e = 0; e < 8; e++) t[e] = *reinterpret_cast<const v4f*>(p + min(s + e, P.splits - 1) * total);
+        for (uint32_t e = 0; e < 8; e++) t[e] = *reinterpret_cast<const v4f*>(p + min(s + e, splits - 1) * total);
 #pragma unroll
         for (uint32_t e = 0; e < 8; e++)
-            if (s + e < P.splits) v += t[e];
+            if (s + e < splits) v += t[e];
     }
     const uint32_t t = (uint32_t)(i / A.N), n = (uint32_t)(i % A.N);
 #pragma unroll
@@ -460,9 +459,12 @@ bool int4_gemm(const nerve_hip_ctx* ctx, const Int4Args& A, const PpArgs* i8, bo
         if (ct) launch_seg<2, true>(P, mt, st);
         else launch_seg<2, false>(P, mt, st);
     }
-    if (P.splits > 1)
-        int4_split_sum_kernel<<<(uint32_t)(((uint64_t)A.B * A.N / 4 + 255) / 256), 256, 0, st>>>(P);
+    if (P.splits > 1) int4_split_sum(A, P.part, P.splits, st);
     return true;
+}
+
+void int4_split_sum(const Int4Args& A, const float* part, uint32_t splits, hipStream_t st) {
+    int4_split_sum_kernel<<<(uint32_t)(((uint64_t)A.B * A.N / 4 + 255) / 256), 256, 0, st>>>(A, part, splits);
 }
 
 }  // namespace nh

@@ -321,7 +321,6 @@ __global__ __launch_bounds__(64 * NW, WPE) void sparse_tile_kernel(SmArgs A, uin
     constexpr uint32_t NL = 16 * PP / 64;                               // weight loads per lane, row tile and panel
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     __shared__ uint32_t t_route[TS], t_word[TS];
-    __shared__ uint32_t t_count;
     const uint32_t K = A.K, N = A.N, ng = K / A.G, nblk = K / 32;   // G = 32 << gshift
     const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const uint32_t g = lane >> 4, rr = lane & 15;

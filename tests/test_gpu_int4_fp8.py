@@ -258,6 +258,19 @@ def test_int4_cooperative_batch64(ctx, dev, B, layout, G, finalize):
     assert ok and exact > 0.9, (worst, exact)
 
 
+# Decode forms: the split GPTQ linears (K / 256 > 16: more than one batch per
+# wave, a last split with fewer), the split-K form below 17 rows, and the CT
+# kernel at one and two row tiles a block, a K range that ends inside a batch,
+# waves without steps and a second token tile (scales off 8 bytes).
+@pytest.mark.parametrize("layout,M,K,N,G,asym", [
+    ("gptq", 1, 8192, 64, 128, True), ("gptq", 4, 9216, 128, 32, False), ("gptq", 3, 4608, 64, 256, True),
+    ("gptq", 5, 8192, 64, 64, True), ("gptq", 16, 6400, 192, 128, False), ("ct", 1, 128, 16, 128, False),
+    ("ct", 2, 1664, 8192, 128, False), ("ct", 3, 1664, 8192, 128, False), ("ct", 16, 5376, 48, 256, False),
+    ("ct", 20, 4352, 32, 128, False)])
+def test_int4_decode_forms(ctx, dev, layout, M, K, N, G, asym):
+    test_int4_linear_tiles(ctx, dev, layout, M, K, N, G, asym)
+
+
 # The tiled split-K form (more than 16 rows): row tiles 1..4 with remainders,
 # column tiles cut at 16 and at 256, K tails of half a stage, scale segments of
 # 1, 2 and 4 blocks (G = 96 falls back to one), with and without zero points,
