@@ -1854,8 +1854,8 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
 
 // Fused set-up tables (in the LDS ring, before any copy is issued).
 constexpr uint32_t FUSED_MAX_EXPERTS = 512;
-constexpr uint32_t FUSED_MAX_SLOTS = 1024;
 constexpr uint32_t FUSED_MAX_WAVES = 8;
+constexpr uint32_t FUSED_MAX_SLOTS = 64 * FUSED_MAX_WAVES;   // a thread per compacted slot
 
 // A block's whole work as the one-wave set-up publishes it: the tile's
 // parameter pointers, its route ids and words, and the block's row-block
@@ -1877,6 +1877,7 @@ struct FusedTables {
     uint32_t rtab[FUSED_MAX_SLOTS];       // route word of route index r
     uint16_t eslot[FUSED_MAX_SLOTS];      // its expert (NO_EXPERT: skipped)
     uint16_t rank[FUSED_MAX_SLOTS];       // its position among its expert's slots
+    uint64_t wcnt[FUSED_MAX_EXPERTS];     // byte w: valid routes of the expert among wave w's slots
     uint8_t valid[FUSED_MAX_EXPERTS];
     uint32_t wlist[FUSED_MAX_WAVES][16];  // per wave: slots of the tile being set up
 };
@@ -1886,12 +1887,17 @@ struct FusedTables {
 // itself (the same rules as build_tiles: invalid parameters or expert ids
 // skip a route; 16 routes per tile).  One round of independent global loads
 // (slot words, route map, route words, control words and the whole address
-// table, copied into LDS after the tables), then LDS work.  Each slot's rank
-// among its expert's slots comes from the counting atomic.  The launch has a
+// table, copied into LDS after the tables), then LDS work.  The launch has a
 // thread per expert and per compacted slot.
+//
+// A slot's rank among its expert's slots is its place in slot order: every block
+// has to come to the same tiles, so ranks do not depend on the order in which
+// its waves arrive.  A wave ranks its own 64 slots by ballots over the expert's
+// bits and leaves its count per expert; the counts of the waves before are added
+// after a barrier.
 template <int NW>
 __device__ __forceinline__ void fused_tables(const TileArgs& A, FusedTables& F, uint32_t* addr_lds) {
-    static_assert(NW <= (int)FUSED_MAX_WAVES, "per-wave lists");
+    static_assert(NW <= (int)FUSED_MAX_WAVES, "per-wave lists and counts");
     const uint32_t tid = threadIdx.x, nt = 64 * NW;
     const uint32_t cap = A.batch_width * A.k, P = A.P;
     uint32_t sl[4] = {UNBOUND_SLOT, UNBOUND_SLOT, UNBOUND_SLOT, UNBOUND_SLOT};
@@ -1933,17 +1939,39 @@ __device__ __forceinline__ void fused_tables(const TileArgs& A, FusedTables& F, 
             F.eptr[tid][p] = (uint64_t)rec[0] | ((uint64_t)rec[1] << 32);
         }
         F.valid[tid] = ok ? 1 : 0;
-        F.cnt[tid] = 0;
+        F.wcnt[tid] = 0;
     }
     uint32_t n = c2 != 0u ? c3 : cap;
     if (n > cap) n = cap;
     __syncthreads();
-    for (uint32_t c = tid; c < cap; c += nt) {
-        const uint32_t r = F.rw[c], w = r < cap ? F.rtab[r] : 0u, e = w & 0xffffu;
-        F.rword[c] = w;
-        const bool ok = c < n && r < cap && e < A.E && F.valid[e];
-        F.eslot[c] = ok ? (uint16_t)e : NO_EXPERT;
-        if (ok) F.rank[c] = (uint16_t)atomicAdd(&F.cnt[e], 1u);
+    const uint32_t lane = tid & 63, wave = tid >> 6;
+    const uint32_t r = tid < cap ? r0 : cap, w = r < cap ? F.rtab[r] : 0u, e = w & 0xffffu;
+    const bool ok = tid < n && r < cap && e < A.E && F.valid[e];
+    uint64_t same = __ballot(ok);
+#pragma unroll
+    for (uint32_t bit = 0; bit < 9; bit++) {           // E <= FUSED_MAX_EXPERTS
+        const uint64_t m = __ballot(ok && ((e >> bit) & 1u));
+        same &= ((e >> bit) & 1u) ? m : ~m;
+    }
+    uint32_t rank = (uint32_t)__popcll(same & ((1ull << lane) - 1ull));
+    if (ok && rank == 0) reinterpret_cast<uint8_t*>(&F.wcnt[e])[wave] = (uint8_t)__popcll(same);
+    __syncthreads();
+    if (tid < A.E) {
+        const uint64_t all = F.wcnt[tid];
+        uint32_t total = 0;
+#pragma unroll
+        for (uint32_t b = 0; b < FUSED_MAX_WAVES; b++) total += (uint32_t)(all >> (8 * b)) & 0xffu;
+        F.cnt[tid] = total;
+    }
+    if (ok) {
+        const uint64_t before = F.wcnt[e] & ((1ull << (8 * wave)) - 1ull);
+#pragma unroll
+        for (uint32_t b = 0; b < FUSED_MAX_WAVES; b++) rank += (uint32_t)(before >> (8 * b)) & 0xffu;
+    }
+    if (tid < cap) {
+        F.rword[tid] = w;
+        F.eslot[tid] = ok ? (uint16_t)e : NO_EXPERT;
+        F.rank[tid] = (uint16_t)rank;
     }
     __syncthreads();
 }
@@ -1961,7 +1989,7 @@ __device__ __forceinline__ uint32_t fused_tile_scan(const FusedTables& F, uint32
     tk = 0;
     for (uint32_t e0 = 0; e0 < E; e0 += 64) {
         const uint32_t e = e0 + lane;
-        const uint32_t nte = e < E ? (F.cnt[e] + 15u) / 16u : 0u;   // <= 64 (slots <= 1024)
+        const uint32_t nte = e < E ? (F.cnt[e] + 15u) / 16u : 0u;   // <= 32 (slots <= 512)
         uint32_t excl = 0, tot = 0;
 #pragma unroll
         for (uint32_t bit = 0; bit < 7; bit++) {
@@ -2277,7 +2305,7 @@ nerve_hip_status launch_stream(StreamArgs A, const nerve_hip_ctx* ctx, hipStream
         // Every compacted slot needs a thread in the tables, and activation
         // rows are read in 16-byte pieces.
         const uint32_t cap = A.T.batch_width * A.T.k;
-        if (cap > 64 * NW || cap > FUSED_MAX_SLOTS || A.T.E > FUSED_MAX_EXPERTS || A.T.E > 64 * NW || A.T.P > 4 ||
+        if (cap > 64 * NW || A.T.E > FUSED_MAX_EXPERTS || A.T.E > 64 * NW || A.T.P > 4 ||
             ((uintptr_t)A.x16 & 15) || A.x_frame % 8 || A.x_seg % 8 ||
             (A.T.n_records > A.addr_lds_records && !A.small_plan) ||   // the small plan reads a big table from memory
             ((uintptr_t)A.T.addr & 15))

@@ -234,6 +234,34 @@ def test_prefill_route_count_groups(ctx, dev, counts):
     assert ok and exact > 0.9, (worst, exact)
 
 
+@pytest.mark.parametrize("E,top,B", [(8, 16, 24), (8, 90, 128), (100, 17, 40), (300, 101, 127), (512, 128, 128)])
+def test_decode_experts_of_several_tiles(ctx, dev, E, top, B):
+    """65 to 512 routes, every block building its own tables: an expert of `top`
+    routes spread over all waves' slots has several 16-route tiles, which every
+    block has to split alike (each route in one tile, for every row block)."""
+    k, H, I = 4, 512, 1664
+    rng = np.random.default_rng(1000 * E + top)
+    ex = np.stack([1 + rng.permutation(E - 1)[:k] for _ in range(B)])
+    for t in rng.permutation(B)[:top]:
+        ex[t, rng.integers(k)] = 0
+    d = wl.moe_experts(rng, E, H, I)
+    d["limit"] = 7.0
+    routes = _route_words(ex, rng.uniform(0.05, 1.0, (B, k)).astype(np.float32))
+    hidden = wl.bf16_normal(rng, (B, H))
+    rig = MoeRig(dev, d, routes)
+    cmap, _ = oracle.route_compact(routes, k, (I + 31) // 32, B)
+    h_ref = oracle.moe_gate_up(hidden, routes, cmap, B * k, k, d["gate_w"], d["gate_s"], d["up_w"], d["up_s"], 7.0)
+    h_atol = moe_gate_up_atol(hidden, routes, d["gate_w"], d["gate_s"], d["up_w"], d["up_s"], 7.0)
+    for _ in range(3):
+        rig.run(ctx, hidden)
+        ok, worst, exact = bf16_close(rig.h_np(), h_ref, atol=h_atol, name="decode gate_up")
+        assert ok and exact > 0.9, (worst, exact)
+        eo_ref = oracle.moe_down(rig.h_np(), routes, cmap, B * k, d["down_w"], d["down_s"])
+        ok, worst, exact = bf16_close(to_np(rig.expert_out, np.uint16), eo_ref,
+                                      atol=moe_down_atol(rig.h_np(), routes, d["down_w"], d["down_s"]), name="decode down")
+        assert ok and exact > 0.9, (worst, exact)
+
+
 # H = 128: the span kernels; H = 512: the token-form gate_up kernel and the
 # streaming down kernel.
 @pytest.mark.parametrize("H,I", [(128, 128), (512, 256)])
