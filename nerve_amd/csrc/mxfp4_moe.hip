@@ -1388,7 +1388,7 @@ struct StreamArgs {
     uint16_t* out16;
     uint64_t frame_elems;
     float limit;
-    uint32_t w_region, s_region, slot_bytes;   // LDS layout of one ring slot
+    uint32_t w_stride, w_region, s_region, slot_bytes;   // LDS layout of one ring slot
     uint32_t lw, ls;                            // copies per wave per matrix (weights, scales)
     uint32_t copies_per_item;                   // per wave: NMAT * (lw + ls)
     // Fused set-up (no preparation launch): the route map and parameter
@@ -1411,6 +1411,13 @@ struct StreamArgs {
     // ((q / 4) N + r) 4 + q % 4.
     uint32_t block_major;
 };
+
+// LDS bytes from one weight row to the next.  With K % 128 == 0 the operand
+// reads of 16 rows fall on one or two groups of banks (K = 2048 and 1536, 96
+// routes over 64 experts: gate_up 71.7 us, down 40.5), with 16 bytes between
+// them on distinct ones (47.4, 29.0).  Other K spread the rows already, and
+// there the gap costs 2 %.
+inline uint32_t lds_row_stride(uint32_t K) { return K / 2 + (K % 128 == 0 ? 16 : 0); }
 
 // One tile as the streaming loop sees it: its parameter pointers, its route
 // count, and per lane the route whose activations it loads (row rr) and the
@@ -1518,7 +1525,9 @@ __device__ __forceinline__ uint32_t sload_u32(const uint32_t* p) {
 // One contiguous range of work items [i0, i1) of one tile, run by NW waves
 // that split each item's K chunks.  An item is RI = 16 NSUB rows of each of
 // the NMAT matrices.
-template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool FUSED>
+// QIN: the activation rows are e4m3 with pow2 block scales (A.aq, A.as); bf16
+// rows (A.x16) are quantized in registers otherwise.
+template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool QIN>
 __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, uint32_t i1, uint32_t nrb,
                                              const TileSrc& ts) {
     constexpr uint32_t RI = 16 * NSUB;
@@ -1566,6 +1575,14 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
 #pragma unroll
     for (uint32_t t = 0; t < LWMAX; t++)
         wsrc[t] = A.block_major ? ((woff[t] % RB) / 64) * N * 64 + (woff[t] / RB) * 64 + woff[t] % 64 : woff[t];
+    // LDS offsets: rows A.w_stride apart (a 16-byte piece never straddles a row).
+    uint32_t wdst[LWMAX];
+#pragma unroll
+    for (uint32_t t = 0; t < LWMAX; t++) wdst[t] = woff[t];
+    if (A.w_stride != RB) {                       // no division for the rows that need no padding
+#pragma unroll
+        for (uint32_t t = 0; t < LWMAX; t++) wdst[t] += woff[t] / RB * (A.w_stride - RB);
+    }
 #pragma unroll
     for (uint32_t t = 0; t < LSMAX; t++)
         ssrc[t] = A.block_major ? ((soff[t] % SB) / 4) * N * 4 + (soff[t] / SB) * 4 : soff[t];
@@ -1602,7 +1619,7 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
         for (int m = 0; m < NMAT; m++) {
 #pragma unroll
             for (uint32_t t = 0; t < LWMAX; t++)
-                if (t < lw) *reinterpret_cast<v4i*>(dst + m * A.w_region + woff[t]) = R.w[m][t];
+                if (t < lw) *reinterpret_cast<v4i*>(dst + m * A.w_region + wdst[t]) = R.w[m][t];
 #pragma unroll
             for (uint32_t t = 0; t < LSMAX; t++)
                 if (t < ls) *reinterpret_cast<uint32_t*>(dst + NMAT * A.w_region + m * A.s_region + soff[t]) = R.s[m][t];
@@ -1619,7 +1636,7 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
         const uint32_t c = c0 + q, kb = c * 128 + g * 32;
         kvalid[q] = c < c1 && kb < K;
         const uint32_t kk = kvalid[q] ? kb : 0;
-        rw[q] = rr * RB + kk / 2;
+        rw[q] = rr * A.w_stride + kk / 2;
         rs[q] = NMAT * A.w_region + rr * SB + kk / 32;
     }
 
@@ -1632,7 +1649,7 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
     v8i av[CH];
     uint32_t sa[CH];
     v4i lo[CH], hi[CH];          // e4m3 operand halves (pre-quantized input)
-    float sraw[CH];
+    uint32_t sraw[CH];
     v4i xb[CH][4];               // bf16 operand halves (fused quantization)
     // Which of this lane's activation pieces exist (k0 < K covers a whole
     // 16-column half since K % 32 == 0).
@@ -1641,7 +1658,7 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
         return arow_ok && c < c1 && k0 < K;
     };
     auto act_request = [&]() __attribute__((always_inline)) {
-        if (FUSED) {
+        if (!QIN) {
             // Inline-asm loads: the compiler does not count them, so it adds
             // no wait for them in front of the weight copies issued next.
             // Every piece is loaded (absent ones from the row start, which
@@ -1658,24 +1675,21 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
                 }
             }
         } else {
-            const uint32_t row = ts.in_route / A.a_row_div;
-            const uint8_t* arow = A.aq + (uint64_t)(arow_ok ? row : 0) * K;
-            const float* ascale = A.as + (uint64_t)(arow_ok ? row : 0) * nch;
+            const uint32_t row = arow_ok ? ts.in_route / A.a_row_div : 0u;
+            const uint8_t* arow = A.aq + (uint64_t)row * K;
+            const float* ascale = A.as + (uint64_t)row * nch;
 #pragma unroll
             for (uint32_t q = 0; q < CH; q++) {
-                const uint32_t c = c0 + q, k0 = c * 128 + g * 16;
-                lo[q] = hi[q] = v4i{0, 0, 0, 0};
-                sraw[q] = 1.0f;
-                if (arow_ok && c < c1) {
-                    if (k0 < K) lo[q] = *reinterpret_cast<const v4i*>(arow + k0);
-                    if (k0 + 64 < K) hi[q] = *reinterpret_cast<const v4i*>(arow + k0 + 64);
-                    sraw[q] = ascale[c];
-                }
+                if (c0 + q >= c1) continue;
+                const uint32_t k0 = (c0 + q) * 128 + g * 16;
+                lo[q] = gload16_untracked(arow + (piece_ok(q, 0) ? k0 : 0u));
+                hi[q] = gload16_untracked(arow + (piece_ok(q, 2) ? k0 + 64u : 0u));
+                sraw[q] = gload4_untracked(ascale + c0 + q);
             }
         }
     };
     auto act_finish = [&]() {
-        if (FUSED) {
+        if (!QIN) {
             // Blockwise e4m3 quantization of this lane's 32 values of each
             // 128-column block (the same arithmetic as quant_unit: pow2
             // scale of the block amax, x / scale rounded to e4m3).  The four
@@ -1699,11 +1713,14 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
             }
         } else {
 #pragma unroll
-            for (uint32_t q = 0; q < CH; q++) asm volatile("" : "+v"(lo[q]), "+v"(hi[q]), "+v"(sraw[q]));
-#pragma unroll
             for (uint32_t q = 0; q < CH; q++) {
-                av[q] = v8i{lo[q].x, lo[q].y, lo[q].z, lo[q].w, hi[q].x, hi[q].y, hi[q].z, hi[q].w};
-                sa[q] = arow_ok ? pow2_to_e8m0(sraw[q]) : 127u;
+                av[q] = v8i{0, 0, 0, 0, 0, 0, 0, 0};
+                sa[q] = 127u;
+                if (c0 + q >= c1) continue;
+                asm volatile("" : "+v"(lo[q]), "+v"(hi[q]), "+v"(sraw[q]));
+                const v4i l = piece_ok(q, 0) ? lo[q] : v4i{0, 0, 0, 0}, h = piece_ok(q, 2) ? hi[q] : v4i{0, 0, 0, 0};
+                av[q] = v8i{l.x, l.y, l.z, l.w, h.x, h.y, h.z, h.w};
+                if (arow_ok) sa[q] = pow2_to_e8m0(__uint_as_float(sraw[q]));
             }
         }
     };
@@ -1766,7 +1783,7 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
                 for (int m = 0; m < NMAT; m++) {
 #pragma unroll
                     for (int j = 0; j < NSUB; j++) {
-                        w[u][m][j] = lds_read16(buf + m * A.w_region + j * 16 * RB + rw[q0 + u]);
+                        w[u][m][j] = lds_read16(buf + m * A.w_region + j * 16 * A.w_stride + rw[q0 + u]);
                         sw[u][m][j] = lds_read_u8(buf + m * A.s_region + j * 16 * SB + rs[q0 + u]);
                     }
                 }
@@ -2193,7 +2210,7 @@ __device__ __forceinline__ void fused_small_plan(const TileArgs& A, SmallPlan& S
     __syncthreads();
 }
 
-template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool FUSED>
+template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool FUSED, bool QIN>
 __global__ __launch_bounds__(64 * NW) void mx_stream_kernel(StreamArgs A) {
     extern __shared__ __attribute__((aligned(16))) uint8_t ring[];
     if (A.count_control && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -2223,7 +2240,7 @@ __global__ __launch_bounds__(64 * NW) void mx_stream_kernel(StreamArgs A) {
         ts.out_route = ov ? S.route[tl] : 0u;
         ts.out_word = ov ? S.word[tl] : 0u;
         lds_drain();   // the plan is read before any copy can overwrite it
-        stream_range<MODE, NMAT, NBUF, NW, NSUB, FUSED>(A, tile * nrb + lo_rb, tile * nrb + hi_rb, nrb, ts);
+        stream_range<MODE, NMAT, NBUF, NW, NSUB, QIN>(A, tile * nrb + lo_rb, tile * nrb + hi_rb, nrb, ts);
         return;
     }
     if (FUSED) {
@@ -2264,13 +2281,13 @@ __global__ __launch_bounds__(64 * NW) void mx_stream_kernel(StreamArgs A) {
         block_share(G, b, n_tiles, nrb, tile, lo_rb, hi_rb);
         if (lo_rb >= hi_rb) return;
         const TileSrc ts = tile_src(tile);
-        stream_range<MODE, NMAT, NBUF, NW, NSUB, FUSED>(A, tile * nrb + lo_rb, tile * nrb + hi_rb, nrb, ts);
+        stream_range<MODE, NMAT, NBUF, NW, NSUB, QIN>(A, tile * nrb + lo_rb, tile * nrb + hi_rb, nrb, ts);
     } else {
         for (uint32_t t = b; t < n_tiles; t += G) {
             // The tables share LDS with the ring: rebuild them after a range.
             if (FUSED && t != b) fused_tables<NW>(A.T, F, addr_lds);
             const TileSrc ts = tile_src(t);
-            stream_range<MODE, NMAT, NBUF, NW, NSUB, FUSED>(A, t * nrb, (t + 1) * nrb, nrb, ts);
+            stream_range<MODE, NMAT, NBUF, NW, NSUB, QIN>(A, t * nrb, (t + 1) * nrb, nrb, ts);
         }
     }
 }
@@ -2278,15 +2295,16 @@ __global__ __launch_bounds__(64 * NW) void mx_stream_kernel(StreamArgs A) {
 // Launches the streaming kernel, or returns UNSUPPORTED when the shape does
 // not fit its LDS ring or copy-count limits (the caller then uses the span
 // kernel).
-template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool FUSED>
+template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool FUSED, bool QIN>
 nerve_hip_status launch_stream(StreamArgs A, const nerve_hip_ctx* ctx, hipStream_t st) {
     constexpr uint32_t RI = 16 * NSUB;
     // Spans of at least one 1 KB weight piece and one 256 B scale piece.
     if (A.K > 4096 || A.K % 32 || RI * (A.K / 32) < 256) return NERVE_HIP_UNSUPPORTED;
-    A.w_region = RI * (A.K / 2);
+    A.w_stride = lds_row_stride(A.K);
+    A.w_region = RI * A.w_stride;
     A.s_region = RI * (A.K / 32);
     A.slot_bytes = NMAT * (A.w_region + A.s_region);
-    const uint32_t npw = (A.w_region + 1023) / 1024, nps = (A.s_region + 255) / 256;
+    const uint32_t npw = (RI * (A.K / 2) + 1023) / 1024, nps = (A.s_region + 255) / 256;
     A.lw = (npw + NW - 1) / NW;
     A.ls = (nps + NW - 1) / NW;
     A.copies_per_item = NMAT * (A.lw + A.ls);
@@ -2302,23 +2320,24 @@ nerve_hip_status launch_stream(StreamArgs A, const nerve_hip_ctx* ctx, hipStream
     A.addr_lds_records = FUSED ? (uint32_t)((lds - head) / 32) : 0u;
     if (lds > 160 * 1024 || A.copies_per_item * 2 > 63) return NERVE_HIP_UNSUPPORTED;
     if (FUSED) {
-        // Every compacted slot needs a thread in the tables, and activation
-        // rows are read in 16-byte pieces.
+        // Every compacted slot needs a thread in the tables.  Activation rows
+        // are read in 16-byte pieces at any dword: a frame of k I / 2 + k words
+        // starts off 16 bytes unless k % 4 == 0.
         const uint32_t cap = A.T.batch_width * A.T.k;
         if (cap > 64 * NW || A.T.E > FUSED_MAX_EXPERTS || A.T.E > 64 * NW || A.T.P > 4 ||
-            ((uintptr_t)A.x16 & 15) || A.x_frame % 8 || A.x_seg % 8 ||
+            ((uintptr_t)A.x16 & 3) || A.x_frame % 2 || A.x_seg % 2 ||
             (A.T.n_records > A.addr_lds_records && !A.small_plan) ||   // the small plan reads a big table from memory
             ((uintptr_t)A.T.addr & 15))
             return NERVE_HIP_UNSUPPORTED;
     }
     static bool attr_set = false;
     if (!attr_set) {
-        if (hipFuncSetAttribute((const void*)mx_stream_kernel<MODE, NMAT, NBUF, NW, NSUB, FUSED>,
+        if (hipFuncSetAttribute((const void*)mx_stream_kernel<MODE, NMAT, NBUF, NW, NSUB, FUSED, QIN>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
             return nh::fail(NERVE_HIP_DEVICE_ERROR, "hipFuncSetAttribute failed for mx_stream_kernel");
         attr_set = true;
     }
-    mx_stream_kernel<MODE, NMAT, NBUF, NW, NSUB, FUSED><<<ctx->cu_count, 64 * NW, lds, st>>>(A);
+    mx_stream_kernel<MODE, NMAT, NBUF, NW, NSUB, FUSED, QIN><<<ctx->cu_count, 64 * NW, lds, st>>>(A);
     return nh::check_launch("mx_stream_kernel");
 }
 
@@ -2561,6 +2580,13 @@ __device__ __forceinline__ void mx_tokens_body(const StreamArgs& A) {
         spos[q] = min(pc * 256, RI * SB - 256);
         soff[q] = spos[q] + lane * 4;
     }
+    uint32_t wdst[LWMAX];                     // LDS offsets: rows A.w_stride apart
+#pragma unroll
+    for (uint32_t q = 0; q < LWMAX; q++) wdst[q] = woff[q];
+    if (A.w_stride != RB) {
+#pragma unroll
+        for (uint32_t q = 0; q < LWMAX; q++) wdst[q] += woff[q] / RB * (A.w_stride - RB);
+    }
     // Item i: expert index i / nrb (u0 or u0 + 1), rows (i % nrb) * 16.
     // Its weight and scale bytes are loaded with nontemporal loads into a
     // register set (the same 1 KB / 256 B pieces per wave as a ring slot's
@@ -2594,7 +2620,7 @@ __device__ __forceinline__ void mx_tokens_body(const StreamArgs& A) {
         for (uint32_t m = 0; m < NMAT; m++) {
 #pragma unroll
             for (uint32_t q = 0; q < LWMAX; q++)
-                if (q < lw) *reinterpret_cast<v4i*>(dst + m * A.w_region + woff[q]) = R.w[m][q];
+                if (q < lw) *reinterpret_cast<v4i*>(dst + m * A.w_region + wdst[q]) = R.w[m][q];
 #pragma unroll
             for (uint32_t q = 0; q < LSMAX; q++)
                 if (q < ls) *reinterpret_cast<uint32_t*>(dst + NMAT * A.w_region + m * A.s_region + soff[q]) = R.s[m][q];
@@ -2607,7 +2633,7 @@ __device__ __forceinline__ void mx_tokens_body(const StreamArgs& A) {
         const uint32_t c = c0 + q, kb = c * 128 + g * 32;
         kvalid[q] = c < c1 && kb < K;
         const uint32_t kk = kvalid[q] ? kb : 0;
-        rw[q] = rr * RB + kk / 2;
+        rw[q] = rr * A.w_stride + kk / 2;
         rs[q] = NMAT * A.w_region + rr * SB + kk / 32;
     }
 
@@ -2769,10 +2795,11 @@ nerve_hip_status launch_tokens(StreamArgs A, const nerve_hip_ctx* ctx, hipStream
         ((uintptr_t)A.x16 & 15) || A.x_frame % 8 || ((uintptr_t)A.T.addr & 15) || A.T.k > 32 ||
         (uint32_t)ctx->cu_count < A.T.E)   // >= E blocks: a block's share spans at most two experts
         return NERVE_HIP_UNSUPPORTED;
-    A.w_region = RI * (A.K / 2);
+    A.w_stride = lds_row_stride(A.K);
+    A.w_region = RI * A.w_stride;
     A.s_region = RI * (A.K / 32);
     A.slot_bytes = 2 * (A.w_region + A.s_region);
-    const uint32_t npw = (A.w_region + 1023) / 1024, nps = (A.s_region + 255) / 256;
+    const uint32_t npw = (RI * (A.K / 2) + 1023) / 1024, nps = (A.s_region + 255) / 256;
     A.lw = (npw + NW - 1) / NW;
     A.ls = (nps + NW - 1) / NW;
     A.copies_per_item = 2 * (A.lw + A.ls);
@@ -4514,14 +4541,13 @@ static nerve_hip_status moe_common(nerve_hip_ctx* ctx, const nh::MoeSpec& ms, bo
             fa.x_seg = 0;
             fa.out16 = static_cast<uint16_t*>(intermediates);
             if (ms.prequant) {
-                // Only the token form reads prequantized rows in its fused
-                // set-up; other decode shapes take the preparation launch.
                 fa.aq = static_cast<const uint8_t*>(pre_q);
                 fa.as = static_cast<const float*>(pre_s);
                 st = launch_tokens<3, 8>(fa, ctx, stream);
+                if (st == NERVE_HIP_UNSUPPORTED) st = launch_stream<SPAN_GATE_UP, 2, 3, 8, 1, true, true>(fa, ctx, stream);
             } else {
                 st = launch_tokens<3, 8>(fa, ctx, stream);
-                if (st == NERVE_HIP_UNSUPPORTED) st = launch_stream<SPAN_GATE_UP, 2, 3, 8, 1, true>(fa, ctx, stream);
+                if (st == NERVE_HIP_UNSUPPORTED) st = launch_stream<SPAN_GATE_UP, 2, 3, 8, 1, true, false>(fa, ctx, stream);
             }
         } else {
             fa.x16 = frames16;
@@ -4531,7 +4557,7 @@ static nerve_hip_status moe_common(nerve_hip_ctx* ctx, const nh::MoeSpec& ms, bo
             fa.count_control = count_control;
             fa.count_tiles = (H + 63) / 64;
             fa.block_major = ms.input_block_major ? 1u : 0u;
-            st = launch_stream<SPAN_DOWN, 1, 3, 8, 2, true>(fa, ctx, stream);
+            st = launch_stream<SPAN_DOWN, 1, 3, 8, 2, true, false>(fa, ctx, stream);
             if (st == NERVE_HIP_OK) count_control = nullptr;
         }
         if (st != NERVE_HIP_UNSUPPORTED) return st;
@@ -4675,12 +4701,12 @@ static nerve_hip_status moe_common(nerve_hip_ctx* ctx, const nh::MoeSpec& ms, bo
         qa.limit = ea.limit;
         if (gate_up) {
             sa.out16 = qa.out16 = static_cast<uint16_t*>(intermediates);
-            st = launch_stream<SPAN_GATE_UP, 2, 3, 8, 1, false>(qa, ctx, stream);
+            st = launch_stream<SPAN_GATE_UP, 2, 3, 8, 1, false, true>(qa, ctx, stream);
             if (st != NERVE_HIP_UNSUPPORTED) return st;
             return launch_span<SPAN_GATE_UP, 2, 1>(sa, max_tiles, stream);
         }
         sa.out16 = qa.out16 = static_cast<uint16_t*>(expert_outputs);
-        st = launch_stream<SPAN_DOWN, 1, 3, 8, 2, false>(qa, ctx, stream);
+        st = launch_stream<SPAN_DOWN, 1, 3, 8, 2, false, true>(qa, ctx, stream);
         if (st != NERVE_HIP_UNSUPPORTED) return st;
         return launch_span<SPAN_DOWN, 1, 2>(sa, max_tiles, stream);
     }

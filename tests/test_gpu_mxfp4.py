@@ -234,12 +234,16 @@ def test_prefill_route_count_groups(ctx, dev, counts):
     assert ok and exact > 0.9, (worst, exact)
 
 
-@pytest.mark.parametrize("E,top,B", [(8, 16, 24), (8, 90, 128), (100, 17, 40), (300, 101, 127), (512, 128, 128)])
-def test_decode_experts_of_several_tiles(ctx, dev, E, top, B):
+# Frames off 16 bytes (k = 1, 3, 5, 6), rows that need padding in LDS (K % 128 == 0)
+# and not.
+@pytest.mark.parametrize("E,top,B,k,H,I", [(8, 16, 24, 4, 512, 1664), (8, 90, 128, 4, 544, 1664), (100, 17, 40, 4, 512, 800),
+                                           (300, 101, 127, 4, 768, 544), (512, 128, 128, 4, 512, 544),
+                                           (16, 60, 90, 1, 512, 800), (12, 33, 34, 3, 800, 1536),
+                                           (20, 40, 100, 5, 512, 544), (64, 64, 64, 6, 2048, 1536)])
+def test_decode_experts_of_several_tiles(ctx, dev, E, top, B, k, H, I):
     """65 to 512 routes, every block building its own tables: an expert of `top`
     routes spread over all waves' slots has several 16-route tiles, which every
     block has to split alike (each route in one tile, for every row block)."""
-    k, H, I = 4, 512, 1664
     rng = np.random.default_rng(1000 * E + top)
     ex = np.stack([1 + rng.permutation(E - 1)[:k] for _ in range(B)])
     for t in rng.permutation(B)[:top]:
@@ -260,6 +264,16 @@ def test_decode_experts_of_several_tiles(ctx, dev, E, top, B):
         ok, worst, exact = bf16_close(to_np(rig.expert_out, np.uint16), eo_ref,
                                       atol=moe_down_atol(rig.h_np(), routes, d["down_w"], d["down_s"]), name="decode down")
         assert ok and exact > 0.9, (worst, exact)
+    # the same bytes from hidden rows that are quantized already
+    torch = _torch()
+    h, q = rig.h_np(), torch.zeros(B, H, dtype=torch.uint8, device=dev)
+    s = torch.zeros(B, (H + 127) // 128, dtype=torch.float32, device=dev)
+    ctx.quantize_fp8_e4m3(f"quantize_batch{B}_fp8_e4m3_spow2_b128_h{H}.comp", to_dev(hidden, dev), B, q, s)
+    rig.inter.zero_()
+    ctx.moe_route_compact(rig.gu, rig.routes, rig.inter, rig.control, B)
+    ctx.mxfp4_moe_gate_up(gate_up_spec(H, I, E, k, 7.0, prequant=True), q, s, rig.routes, rig.inter, rig.bank.addresses,
+                          rig.bank.gate_slots, rig.control, B)
+    assert np.array_equal(rig.h_np(), h)
 
 
 # H = 128: the span kernels; H = 512: the token-form gate_up kernel and the
