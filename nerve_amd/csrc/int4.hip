@@ -606,15 +606,20 @@ __global__ __launch_bounds__(256) void int4_pp_kernel(PpArgs P) {
 // Bound: the weight stream and, from about 32 tokens on, the activation rows
 // every column tile re-reads from L2.  One token of 4096 x 14336: 11.0 us a
 // launch (31.3 with a lane per column), of 14336 x 4096 13.4 us; a feed-forward
-// of 30 tokens 1782 -> 62 us.
+// of 30 tokens 1782 -> 62 us.  Up to four tokens the conversion and fold of all
+// 16 result rows is the larger part: RT = 1 gives each lane group one token
+// (operand rows 4 t .. 4 t + 3 repeat token t) and folds one row in four: 9.3
+// and 12.0 us.
 // ---------------------------------------------------------------------------
-template <int MT, int J, int KS, int U, int BPG, bool PAIRED, bool CT>
-__global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgroups) {
+template <int MT, int J, int KS, int U, int BPG, bool PAIRED, bool CT, int RT>
+__global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgroups, float* split_part) {
     static_assert(U % 2 == 0 && U % BPG == 0, "a batch holds whole 64-column pairs and scale segments");
     static_assert(!CT || (J == 1 && U % 4 == 0), "CT rows are read 128 columns at a time");
-    constexpr int NV = (16 * MT * U + 63) / 64;       // activation scales per lane and batch
-    __shared__ __attribute__((aligned(16))) float xs[KS][U][16 * MT];
-    __shared__ float part[KS][J][64][4];
+    static_assert(RT == 4 || MT == 1, "one token per lane group: at most four tokens");
+    constexpr int TOK = 4 * RT * MT;                  // tokens of the block
+    constexpr int NV = (TOK * U + 63) / 64;           // activation scales per lane and batch
+    __shared__ __attribute__((aligned(16))) float xs[KS][U][TOK];
+    __shared__ __attribute__((aligned(16))) float part[KS][J][64][RT];
     const Int4Args& A = P.L;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const uint32_t g = lane >> 4, rr = lane & 15, pg = ((g & 1) << 1) | (g >> 1);
@@ -623,11 +628,11 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
     // of a tile read its weights through one L2.
     const uint32_t per_xcd = gridDim.x / 8 / tgroups, seq = blockIdx.x / 8;
     const uint32_t tile = (blockIdx.x % 8) * per_xcd + seq / tgroups;
-    const uint32_t n0 = tile * (16 * J), m0 = (seq % tgroups) * (16 * MT);
+    const uint32_t n0 = tile * (16 * J), m0 = (seq % tgroups) * TOK;
     if (n0 >= N) return;
     constexpr uint32_t UNIT = CT ? 4 : (BPG > 2 ? BPG : 2);
-    const uint32_t units = (nblk + UNIT - 1) / UNIT, per = (units + KS - 1) / KS;
-    const uint32_t b0 = min(nblk, wave * per * UNIT), b1 = min(nblk, b0 + per * UNIT);
+    const uint32_t units = (nblk + UNIT - 1) / UNIT, parts = KS * gridDim.y, per = (units + parts - 1) / parts;
+    const uint32_t b0 = min(nblk, (blockIdx.y * KS + wave) * per * UNIT), b1 = min(nblk, b0 + per * UNIT);
     const uint32_t col = n0 + J * rr;
     const uint32_t ngroups = K / A.G;
 
@@ -640,7 +645,7 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
     const uint8_t* arow[MT];
 #pragma unroll
     for (int m = 0; m < MT; m++)
-        arow[m] = reinterpret_cast<const uint8_t*>(P.q) + (uint64_t)min(m0 + 16 * m + rr, M - 1) * K + 16 * g;
+        arow[m] = reinterpret_cast<const uint8_t*>(P.q) + (uint64_t)min(m0 + 4 * RT * m + rr * RT / 4, M - 1) * K + 16 * g;
     // Loads past the wave's range repeat its last pair; their scales are zero.
     auto load = [&](Batch& B, uint32_t b) __attribute__((always_inline)) {
 #pragma unroll
@@ -677,16 +682,17 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
             B.sx[v] = bb < b1 ? s : 0.0f;
         }
     };
-    v4f acc[MT][J];
+    typedef float rows_t __attribute__((ext_vector_type(RT)));
+    rows_t acc[MT][J];
 #pragma unroll
     for (int m = 0; m < MT; m++)
 #pragma unroll
-        for (int j = 0; j < J; j++) acc[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < J; j++) acc[m][j] = rows_t(0.f);
     auto contract = [&](Batch& B) __attribute__((always_inline)) {
 #pragma unroll
         for (int v = 0; v < NV; v++) {
             const uint32_t i = v * 64 + lane;
-            if (16 * MT * U % 64 == 0 || i < 16 * MT * U) xs[wave][i % U][i / U] = B.sx[v];
+            if (TOK * U % 64 == 0 || i < TOK * U) xs[wave][i % U][i / U] = B.sx[v];
         }
         __builtin_amdgcn_wave_barrier();
         if constexpr (CT) {
@@ -701,7 +707,7 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
                 B.w[u][0] = p[0]; B.w[u + 1][0] = p[1]; B.w[u + 2][0] = q[0]; B.w[u + 3][0] = q[1];
             }
         }
-        v4f ag[MT][J];
+        rows_t ag[MT][J];
 #pragma unroll
         for (int u = 0; u < U; u++) {
             long bw[J];
@@ -729,17 +735,17 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
                 const v4i& v = B.a[m][u / 2];
                 const uint32_t a0 = (uint32_t)(u % 2 ? v.z : v.x), a1 = (uint32_t)(u % 2 ? v.w : v.y);
                 const long av = (long)(((uint64_t)a1 << 32) | a0);
-                const v4f sx = *reinterpret_cast<const v4f*>(&xs[wave][u][16 * m + 4 * g]);
+                const rows_t sx = *reinterpret_cast<const rows_t*>(&xs[wave][u][RT * (4 * m + g)]);
 #pragma unroll
                 for (int j = 0; j < J; j++) {
                     const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bw[j], v4i{0, 0, 0, 0}, 0, 0, 0);
-                    if (u % BPG == 0) ag[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
+                    if (u % BPG == 0) ag[m][j] = rows_t(0.f);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) ag[m][j][i] = fmaf((float)d[i], sx[i], ag[m][j][i]);
+                    for (int i = 0; i < RT; i++) ag[m][j][i] = fmaf((float)d[i], sx[i], ag[m][j][i]);
                     if (u % BPG == BPG - 1) {
                         const float sw = decode_scale(B.sw[u / BPG][j], A.scale_bf16);
 #pragma unroll
-                        for (int i = 0; i < 4; i++) acc[m][j][i] = fmaf(ag[m][j][i], sw, acc[m][j][i]);
+                        for (int i = 0; i < RT; i++) acc[m][j][i] = fmaf(ag[m][j][i], sw, acc[m][j][i]);
                     }
                 }
             }
@@ -762,18 +768,19 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
     // added in wave order.
 #pragma unroll
     for (int m = 0; m < MT; m++) {
-        if (m0 + 16 * m >= M) break;
+        if (m0 + 4 * RT * m >= M) break;
 #pragma unroll
-        for (int j = 0; j < J; j++) *reinterpret_cast<v4f*>(&part[wave][j][lane][0]) = acc[m][j];
+        for (int j = 0; j < J; j++) *reinterpret_cast<rows_t*>(&part[wave][j][lane][0]) = acc[m][j];
         __syncthreads();
-        for (uint32_t i = threadIdx.x; i < 256 * J; i += 64 * KS) {
-            const uint32_t t = i / (16 * J), c = i % (16 * J), tt = m0 + 16 * m + t;
+        for (uint32_t i = threadIdx.x; i < 64 * RT * J; i += 64 * KS) {
+            const uint32_t t = i / (16 * J), c = i % (16 * J), tt = m0 + 4 * RT * m + t;
             if (tt >= M) break;
-            const uint32_t l = (t / 4) * 16 + c / J;
-            float v = part[0][c % J][l][t % 4];
+            const uint32_t l = (t / RT) * 16 + c / J;
+            float v = part[0][c % J][l][t % RT];
 #pragma unroll
-            for (int w = 1; w < KS; w++) v += part[w][c % J][l][t % 4];
-            finalize_store(A, tt, n0 + c, v);
+            for (int w = 1; w < KS; w++) v += part[w][c % J][l][t % RT];
+            if (split_part) split_part[((uint64_t)blockIdx.y * M + tt) * N + n0 + c] = v;
+            else finalize_store(A, tt, n0 + c, v);
         }
         __syncthreads();
     }
@@ -781,25 +788,27 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
 
 // SEG: blocks per scale segment (a divisor of the group's blocks), at most a
 // batch.
-template <int MT, int J, int KS, int U, int SEG>
-void launch_i8_form(const PpArgs& P, bool paired, bool ct, hipStream_t st) {
+template <int MT, int J, int KS, int U, int SEG, int RT = 4>
+void launch_i8_form(const PpArgs& P, bool paired, bool ct, uint32_t splits, float* part, hipStream_t st) {
     constexpr int BPG = SEG < U ? SEG : U;
-    const uint32_t tg = (P.L.B + 16 * MT - 1) / (16 * MT), tiles = P.L.N / (16 * J);
-    const uint32_t grid = (tiles + 7) / 8 * 8 * tg;
-    if (paired) int4_i8_kernel<MT, J, KS, U, BPG, true, false><<<grid, 64 * KS, 0, st>>>(P, tg);
-    else if (!ct) int4_i8_kernel<MT, J, KS, U, BPG, false, false><<<grid, 64 * KS, 0, st>>>(P, tg);
-    else if constexpr (J == 1) int4_i8_kernel<MT, J, KS, U, BPG, false, true><<<grid, 64 * KS, 0, st>>>(P, tg);
+    const uint32_t tg = (P.L.B + 4 * RT * MT - 1) / (4 * RT * MT), tiles = P.L.N / (16 * J);
+    const dim3 grid((tiles + 7) / 8 * 8 * tg, splits);
+    if (paired) int4_i8_kernel<MT, J, KS, U, BPG, true, false, RT><<<grid, 64 * KS, 0, st>>>(P, tg, part);
+    else if (!ct) int4_i8_kernel<MT, J, KS, U, BPG, false, false, RT><<<grid, 64 * KS, 0, st>>>(P, tg, part);
+    else if constexpr (J == 1) int4_i8_kernel<MT, J, KS, U, BPG, false, true, RT><<<grid, 64 * KS, 0, st>>>(P, tg, part);
 }
 
 template <int SEG>
-void launch_i8_shape(const PpArgs& P, bool paired, bool ct, uint32_t j, hipStream_t st) {
-    const uint32_t mt = (P.L.B + 15) / 16;
+void launch_i8_shape(const PpArgs& P, bool paired, bool ct, uint32_t j, uint32_t mt, uint32_t splits, float* part, hipStream_t st) {
     if (j == 4) {
-        if (mt == 1) launch_i8_form<1, 4, 8, 8, SEG>(P, paired, ct, st);
-        else launch_i8_form<2, 4, 8, 4, SEG>(P, paired, ct, st);
+        if (P.L.B <= 4) launch_i8_form<1, 4, 8, 8, SEG, 1>(P, paired, ct, splits, part, st);
+        else if (mt == 1) launch_i8_form<1, 4, 8, 8, SEG>(P, paired, ct, splits, part, st);
+        else if (mt == 3) launch_i8_form<3, 4, 8, 4, SEG>(P, paired, ct, splits, part, st);
+        else launch_i8_form<2, 4, 8, 4, SEG>(P, paired, ct, splits, part, st);
     } else {
-        if (mt == 1) launch_i8_form<1, 1, 8, 16, SEG>(P, paired, ct, st);
-        else launch_i8_form<2, 1, 8, 8, SEG>(P, paired, ct, st);
+        if (P.L.B <= 4) launch_i8_form<1, 1, 8, 16, SEG, 1>(P, paired, ct, splits, part, st);
+        else if (mt == 1) launch_i8_form<1, 1, 8, 16, SEG>(P, paired, ct, splits, part, st);
+        else launch_i8_form<2, 1, 8, 8, SEG>(P, paired, ct, splits, part, st);
     }
 }
 
@@ -808,17 +817,33 @@ void launch_i8_shape(const PpArgs& P, bool paired, bool ct, uint32_t j, hipStrea
 // for CT rows); false otherwise (int4_pp_kernel takes every other shape).
 // 64-column tiles (16 bytes a lane) where they fill more than half of the CUs,
 // else 16-column ones: at N = 4096 the 64 wide tiles would stream 29 MB through
-// 64 CUs, and a CU takes in about 27 GB/s.
-bool launch_i8(const PpArgs& P, bool paired, bool ct, int cus, hipStream_t st) {
+// 64 CUs, and a CU takes in about 27 GB/s.  17 to 32 rows take wide tiles there
+// too, K split over the CUs and the partial sums added by a second launch: 14336
+// x 4096 between two 4096 x 14336, 16 / 20 / 32 rows 49.5 / 57.8 / 62.8 us ->
+// 46.1 / 53.8 / 56.6, but 9 rows of smaller shapes lose 2 to 5 %.
+// one_group: up to 48 rows as one group, wide unsplit tiles only past 32 rows.
+bool launch_i8(const PpArgs& P, bool paired, bool ct, bool one_group, const nerve_hip_ctx* ctx, hipStream_t st) {
     const Int4Args& A = P.L;
+    const uint32_t cus = (uint32_t)ctx->cu_count;
     if (A.N % 16 || A.K % 64 || ((uintptr_t)P.q & 15) || ((uintptr_t)A.qw & 15)) return false;
     if (ct && A.K % 128) return false;
-    const uint32_t tg = (A.B + 31) / 32;
-    const uint32_t j = !ct && A.N % 64 == 0 && A.N / 64 * tg * 2 > (uint32_t)cus ? 4 : 1;
-    const uint32_t bpg = A.G % 128 == 0 ? 4 : A.G % 64 == 0 ? 2 : 1;
-    if (bpg == 4) launch_i8_shape<4>(P, paired, ct, j, st);
-    else if (bpg == 2) launch_i8_shape<2>(P, paired, ct, j, st);
-    else launch_i8_shape<1>(P, paired, ct, j, st);
+    const uint32_t mt = A.B <= 16 ? 1 : one_group ? (A.B + 15) / 16 : 2;
+    const uint32_t tg = (A.B + 16 * mt - 1) / (16 * mt), wide = A.N / 64 * tg;
+    const bool can = !ct && A.N % 64 == 0;
+    uint32_t j = can && wide * 2 > cus ? 4 : 1, splits = 1;
+    if (j == 1 && can && mt == 2 && tg == 1) {
+        const uint64_t most = std::min<uint64_t>(A.K / 1024, nh::kSplitBytes / ((uint64_t)A.B * A.N * 4));
+        splits = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(cus / wide, most));
+        if (splits > 1) j = 4;
+    }
+    if (mt > 3 || (mt == 3 && j == 1)) return false;
+    float* part = splits > 1 ? static_cast<float*>(ctx->split) : nullptr;
+    // (three token tiles and two-block segments spill 47 registers)
+    const uint32_t bpg = A.G % 128 == 0 ? 4 : A.G % 64 == 0 && mt < 3 ? 2 : 1;
+    if (bpg == 4) launch_i8_shape<4>(P, paired, ct, j, mt, splits, part, st);
+    else if (bpg == 2) launch_i8_shape<2>(P, paired, ct, j, mt, splits, part, st);
+    else launch_i8_shape<1>(P, paired, ct, j, mt, splits, part, st);
+    if (part) nh::int4_split_sum(A, part, splits, st);
     return true;
 }
 
@@ -1021,11 +1046,14 @@ extern "C" nerve_hip_status nerve_hip_int4_linear_pairpacked(nerve_hip_ctx* ctx,
     P.L.finalize = s.op;
     const uint32_t grid = (s.out + 63) / 64;
     hipStream_t strm = (hipStream_t)stream;
-    // More than 32 rows: the tiled split-K form (48 rows through a 4096 x 14336
-    // feed-forward: 79 us against 88; 30 rows: 66 against 62).
-    if (batch_width > 32 && nh::int4_gemm(ctx, P.L, &P, paired, s.layout == 1, strm))
-        return nh::check_launch("int4_linear_prequant");
-    if (launch_i8(P, paired, s.layout == 1, ctx->cu_count, strm)) return nh::check_launch("int4_linear_prequant");
+    // Up to 32 rows, and 33 to 48 that fill the CUs with 64-column tiles: one
+    // group of rows over the weights (48 rows of 4096 x 14336: 19.7 us against
+    // 25.5; 16-column tiles 33 against 24.5 for 14336 x 4096).  Else the tiled
+    // split-K form.
+    const bool ct = s.layout == 1;
+    if (launch_i8(P, paired, ct, true, ctx, strm)) return nh::check_launch("int4_linear_prequant");
+    if (batch_width > 32 && nh::int4_gemm(ctx, P.L, &P, paired, ct, strm)) return nh::check_launch("int4_linear_prequant");
+    if (launch_i8(P, paired, ct, false, ctx, strm)) return nh::check_launch("int4_linear_prequant");
     if (paired) int4_pp_kernel<true, false><<<grid, 256, 0, strm>>>(P);
     else if (s.layout == 0) int4_pp_kernel<false, false><<<grid, 256, 0, strm>>>(P);
     else int4_pp_kernel<false, true><<<grid, 256, 0, strm>>>(P);

@@ -215,3 +215,14 @@ def test_int4_linear_prequant_tiles(ctx, dev, kind, M, K, N, G):
                                           aux=aux)
     ok, worst, exact = bf16_close(got[:M], ref, atol=linear_atol(x, gptq_dequant(d), finalize), name="prequant tiles")
     assert ok and exact > 0.9, (worst, exact)
+
+
+# One token per lane group (up to four rows, both tile widths, a wave whose batch
+# runs past K), the split wide tiles of 17 to 32 rows (K a few pairs past whole
+# batches; G = 64 and 96) and three token tiles with each segment length.
+@pytest.mark.parametrize("kind", ["paired", "gptq", "ct"])
+@pytest.mark.parametrize("M,K,N,G", [(1, 448, 8256, 64), (3, 2944, 8320, 128), (4, 4160, 96, 32), (17, 2112, 192, 64),
+                                     (32, 3072, 256, 96), (24, 8192, 4160, 128), (33, 448, 8256, 64),
+                                     (48, 1344, 8320, 96), (47, 2048, 8256, 128)])
+def test_int4_linear_prequant_row_groups(ctx, dev, kind, M, K, N, G):
+    test_int4_linear_prequant_tiles(ctx, dev, kind, M, K, N, G)
