@@ -1389,6 +1389,7 @@ struct StreamArgs {
     uint64_t frame_elems;
     float limit;
     uint32_t w_stride, w_region, s_region, slot_bytes;   // LDS layout of one ring slot
+    uint32_t row_magic;                         // umulhi(b, row_magic) = b / (K / 2) for b < 2^17 (K <= 4096)
     uint32_t lw, ls;                            // copies per wave per matrix (weights, scales)
     uint32_t copies_per_item;                   // per wave: NMAT * (lw + ls)
     // Fused set-up (no preparation launch): the route map and parameter
@@ -1578,11 +1579,7 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
     // LDS offsets: rows A.w_stride apart (a 16-byte piece never straddles a row).
     uint32_t wdst[LWMAX];
 #pragma unroll
-    for (uint32_t t = 0; t < LWMAX; t++) wdst[t] = woff[t];
-    if (A.w_stride != RB) {                       // no division for the rows that need no padding
-#pragma unroll
-        for (uint32_t t = 0; t < LWMAX; t++) wdst[t] += woff[t] / RB * (A.w_stride - RB);
-    }
+    for (uint32_t t = 0; t < LWMAX; t++) wdst[t] = woff[t] + __umulhi(woff[t], A.row_magic) * (A.w_stride - RB);
 #pragma unroll
     for (uint32_t t = 0; t < LSMAX; t++)
         ssrc[t] = A.block_major ? ((soff[t] % SB) / 4) * N * 4 + (soff[t] / SB) * 4 : soff[t];
@@ -2301,6 +2298,7 @@ nerve_hip_status launch_stream(StreamArgs A, const nerve_hip_ctx* ctx, hipStream
     // Spans of at least one 1 KB weight piece and one 256 B scale piece.
     if (A.K > 4096 || A.K % 32 || RI * (A.K / 32) < 256) return NERVE_HIP_UNSUPPORTED;
     A.w_stride = lds_row_stride(A.K);
+    A.row_magic = (uint32_t)((1ull << 32) / (A.K / 2)) + 1;
     A.w_region = RI * A.w_stride;
     A.s_region = RI * (A.K / 32);
     A.slot_bytes = NMAT * (A.w_region + A.s_region);
@@ -2582,11 +2580,7 @@ __device__ __forceinline__ void mx_tokens_body(const StreamArgs& A) {
     }
     uint32_t wdst[LWMAX];                     // LDS offsets: rows A.w_stride apart
 #pragma unroll
-    for (uint32_t q = 0; q < LWMAX; q++) wdst[q] = woff[q];
-    if (A.w_stride != RB) {
-#pragma unroll
-        for (uint32_t q = 0; q < LWMAX; q++) wdst[q] += woff[q] / RB * (A.w_stride - RB);
-    }
+    for (uint32_t q = 0; q < LWMAX; q++) wdst[q] = woff[q] + __umulhi(woff[q], A.row_magic) * (A.w_stride - RB);
     // Item i: expert index i / nrb (u0 or u0 + 1), rows (i % nrb) * 16.
     // Its weight and scale bytes are loaded with nontemporal loads into a
     // register set (the same 1 KB / 256 B pieces per wave as a ring slot's
@@ -2796,6 +2790,7 @@ nerve_hip_status launch_tokens(StreamArgs A, const nerve_hip_ctx* ctx, hipStream
         (uint32_t)ctx->cu_count < A.T.E)   // >= E blocks: a block's share spans at most two experts
         return NERVE_HIP_UNSUPPORTED;
     A.w_stride = lds_row_stride(A.K);
+    A.row_magic = (uint32_t)((1ull << 32) / (A.K / 2)) + 1;
     A.w_region = RI * A.w_stride;
     A.s_region = RI * (A.K / 32);
     A.slot_bytes = 2 * (A.w_region + A.s_region);
