@@ -343,7 +343,7 @@ def int4_gemv(args, ctx, dev):
     out = base_line(args, gbs, "GB/s", ms, "bf16xint4->f32",
                     {"workload": f"int4_gptq_g128_asym_m{M}_k4096_n14336", "weight_copies_rotated": copies})
     kname = ("int4_gptq_gemv_kernel<16, 128, true, 1u>" if M == 1 else "int4_gptq_gemv_kernel<16, 128, true, 4u>"
-             if M <= 4 else "int4_gptq_fixed_kernel<16, 4, 4>")
+             if M <= 4 else "int4_gptq_fixed_kernel<16, 4, 4>" if M <= 16 else "int4_gemm_kernel")
     out["roofline"] = {"bound": "hbm", "kernel": kname, "achieved": gbs, "peak": HBM_PEAK_GBS,
                        "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS, "traffic": traffic_for(kname),
                        "algorithmic_bytes_per_launch": alg, "launch_ms": kms}
@@ -409,11 +409,11 @@ def int4_moe(args, ctx, dev):
     dn_gbs = dn_alg / (dn_ms * 1e-3) / 1e9
     out = base_line(args, B * k / (step_ms * 1e-3), "expert-tokens/s", ms, "bf16xint4->f32",
                     {"workload": f"int4_ct_sparse_moe_b{B}_h3072_i1024_e256_k10_g32"})
-    out["roofline"] = {"bound": "hbm", "kernel": "sparse_int4_kernel<true, 32, false> (gate_up)", "achieved": gu_gbs,
+    out["roofline"] = {"bound": "hbm", "kernel": "sparse_tile_kernel (gate_up)", "achieved": gu_gbs,
                        "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gu_gbs / HBM_PEAK_GBS,
-                       "traffic": traffic_for("sparse_int4_kernel<true, 32u, false>"),
+                       "traffic": traffic_for("sparse_tile_kernel<true, 4u, 4u, 256u, 3u, true>"),
                        "algorithmic_bytes_per_launch": gu_alg, "launch_ms": gu_ms}
-    out["down"] = {"kernel": "sparse_int4_kernel<false, 32, false>", "hbm_gbs": dn_gbs, "frac": dn_gbs / HBM_PEAK_GBS,
+    out["down"] = {"kernel": "sparse_tile_kernel (down)", "hbm_gbs": dn_gbs, "frac": dn_gbs / HBM_PEAK_GBS,
                    "algorithmic_bytes_per_launch": dn_alg, "launch_ms": dn_ms}
     out["step_ms_graph"] = step_ms
     return out

@@ -880,9 +880,9 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
     A.scale_bf16 = s.scale_bf16;
     A.finalize = s.op;
     hipStream_t strm = (hipStream_t)stream;
-    // Five rows on, few column tiles and a long K: also the split-K form (16 rows
-    // of 14336 x 4096: 25.4 -> 14.6 us).  More than 16 rows: the tiled split-K form, which expands the weights once
-    // per 64 rows instead of once per 16.  The 16-row kernels stay where one
+    // More than 16 rows: the tiled split-K form, which expands the weights once per
+    // 64 rows instead of once per 16; from five rows on also where column tiles are
+    // few and K is long (16 rows of 14336 x 4096: 25.4 -> 14.6 us).  The 16-row kernels stay where one
     // round of their blocks covers a GPTQ linear with a short K (64 rows of
     // 4096 x 4096: 10.1 against 15.1 us; of 14336 x 4096: 25.9 against 20.0).
     const bool one_round = s.layout == 0 && A.N % 64 == 0 && A.K <= 6144 &&
