@@ -239,8 +239,8 @@ __device__ __forceinline__ float sum8_bf16(v4i v) {
     return s;
 }
 
-template <int KS, int G, bool ZP, uint32_t MT>
-__global__ __launch_bounds__(64 * KS) void int4_gptq_gemv_kernel(Int4Args A, float* split_part) {
+template <int KS, int G, bool ZP, uint32_t MT, bool SPLIT>
+__global__ __launch_bounds__(64 * KS) void int4_gptq_gemv_kernel(Int4Args A, float* split_part, uint32_t span) {
     constexpr uint32_t GR = G / 8;                 // packed rows per group
     constexpr uint32_t GPB = GEMV_ROWS / GR;       // groups per batch
     constexpr uint32_t LR = GEMV_ROWS / 4;         // packed rows per lane per batch
@@ -257,9 +257,9 @@ __global__ __launch_bounds__(64 * KS) void int4_gptq_gemv_kernel(Int4Args A, flo
     if (n0 >= N) return;
     const uint32_t col = n0 + 4 * c;               // first of the lane's 4 columns
     const uint32_t ngroups = K / G;
-    // This split's batches of K (gridDim.y splits), dealt to the waves.
+    // The batches of K, or this split's `span` of them, dealt to the waves.
     const uint32_t batches = (ngroups + GPB - 1) / GPB;
-    const uint32_t s0 = batches * blockIdx.y / gridDim.y, nbatch = batches * (blockIdx.y + 1) / gridDim.y;
+    const uint32_t s0 = SPLIT ? blockIdx.y * span : 0u, nbatch = SPLIT ? min(batches, s0 + span) : batches;
     const uint32_t per = (nbatch - s0 + KS - 1) / KS;
     const uint32_t b0 = min(nbatch, s0 + wave * per), b1 = min(nbatch, b0 + per);
     const uint32_t zshift = 4 * (col % 8);
@@ -340,7 +340,7 @@ __global__ __launch_bounds__(64 * KS) void int4_gptq_gemv_kernel(Int4Args A, flo
         float v = pf[t * 64 + lane];
 #pragma unroll
         for (int w2 = 1; w2 < KS; w2++) v += pf[(w2 * MT + t) * 64 + lane];
-        if (split_part) split_part[((uint64_t)blockIdx.y * M + t) * N + n0 + lane] = v;
+        if (SPLIT) split_part[((uint64_t)blockIdx.y * M + t) * N + n0 + lane] = v;
         else finalize_store(A, t, n0 + lane, v);
     }
 }
@@ -612,7 +612,7 @@ __global__ __launch_bounds__(256) void int4_pp_kernel(PpArgs P) {
 // and 12.0 us.
 // ---------------------------------------------------------------------------
 template <int MT, int J, int KS, int U, int BPG, bool PAIRED, bool CT, int RT>
-__global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgroups, float* split_part) {
+__global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgroups, float* split_part, uint32_t per) {
     static_assert(U % 2 == 0 && U % BPG == 0, "a batch holds whole 64-column pairs and scale segments");
     static_assert(!CT || (J == 1 && U % 4 == 0), "CT rows are read 128 columns at a time");
     static_assert(RT == 4 || MT == 1, "one token per lane group: at most four tokens");
@@ -630,9 +630,9 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
     const uint32_t tile = (blockIdx.x % 8) * per_xcd + seq / tgroups;
     const uint32_t n0 = tile * (16 * J), m0 = (seq % tgroups) * TOK;
     if (n0 >= N) return;
-    constexpr uint32_t UNIT = CT ? 4 : (BPG > 2 ? BPG : 2);
-    const uint32_t units = (nblk + UNIT - 1) / UNIT, parts = KS * gridDim.y, per = (units + parts - 1) / parts;
-    const uint32_t b0 = min(nblk, (blockIdx.y * KS + wave) * per * UNIT), b1 = min(nblk, b0 + per * UNIT);
+    // `per` blocks of K a wave: whole units of a load (CT), an activation pair or a
+    // scale segment.
+    const uint32_t b0 = min(nblk, (blockIdx.y * KS + wave) * per), b1 = min(nblk, b0 + per);
     const uint32_t col = n0 + J * rr;
     const uint32_t ngroups = K / A.G;
 
@@ -793,9 +793,11 @@ void launch_i8_form(const PpArgs& P, bool paired, bool ct, uint32_t splits, floa
     constexpr int BPG = SEG < U ? SEG : U;
     const uint32_t tg = (P.L.B + 4 * RT * MT - 1) / (4 * RT * MT), tiles = P.L.N / (16 * J);
     const dim3 grid((tiles + 7) / 8 * 8 * tg, splits);
-    if (paired) int4_i8_kernel<MT, J, KS, U, BPG, true, false, RT><<<grid, 64 * KS, 0, st>>>(P, tg, part);
-    else if (!ct) int4_i8_kernel<MT, J, KS, U, BPG, false, false, RT><<<grid, 64 * KS, 0, st>>>(P, tg, part);
-    else if constexpr (J == 1) int4_i8_kernel<MT, J, KS, U, BPG, false, true, RT><<<grid, 64 * KS, 0, st>>>(P, tg, part);
+    const uint32_t unit = ct ? 4 : BPG > 2 ? BPG : 2, units = (P.L.K / 32 + unit - 1) / unit;
+    const uint32_t per = (units + KS * splits - 1) / (KS * splits) * unit;
+    if (paired) int4_i8_kernel<MT, J, KS, U, BPG, true, false, RT><<<grid, 64 * KS, 0, st>>>(P, tg, part, per);
+    else if (!ct) int4_i8_kernel<MT, J, KS, U, BPG, false, false, RT><<<grid, 64 * KS, 0, st>>>(P, tg, part, per);
+    else if constexpr (J == 1) int4_i8_kernel<MT, J, KS, U, BPG, false, true, RT><<<grid, 64 * KS, 0, st>>>(P, tg, part, per);
 }
 
 template <int SEG>
@@ -908,20 +910,24 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
             // Few column tiles and more than one batch per wave: K is split so
             // that every CU has a block, the partial sums added by a second
             // launch (14336 x 4096, one row: 64 blocks 14.9 us, 256 10.1).
-            const uint32_t splits = std::max(1u, std::min((A.K / 256 + 15) / 16, (uint32_t)ctx->cu_count / tiles));
+            const uint32_t batches = (A.K / 8 + GEMV_ROWS - 1) / GEMV_ROWS;
+            const uint32_t most = std::max(1u, std::min((A.K / 256 + 15) / 16, (uint32_t)ctx->cu_count / tiles));
+            const uint32_t span = (batches + most - 1) / most, splits = (batches + span - 1) / span;
             float* part = splits > 1 ? static_cast<float*>(ctx->split) : nullptr;
             dim3 g1((tiles + 7) / 8 * 8, splits);
             const bool zp = zeros != nullptr;
-#define NERVE_INT4_GEMV(GG)                                                                   \
-    (batch_width == 1 ? (zp ? int4_gptq_gemv_kernel<16, GG, true, 1><<<g1, 1024, 0, strm>>>(A, part)   \
-                            : int4_gptq_gemv_kernel<16, GG, false, 1><<<g1, 1024, 0, strm>>>(A, part)) \
-                      : (zp ? int4_gptq_gemv_kernel<16, GG, true, 4><<<g1, 1024, 0, strm>>>(A, part)   \
-                            : int4_gptq_gemv_kernel<16, GG, false, 4><<<g1, 1024, 0, strm>>>(A, part)))
+#define NERVE_INT4_GEMV_FORM(GG, ZP, MT)                                                                  \
+    (part ? int4_gptq_gemv_kernel<16, GG, ZP, MT, true><<<g1, 1024, 0, strm>>>(A, part, span)             \
+          : int4_gptq_gemv_kernel<16, GG, ZP, MT, false><<<g1, 1024, 0, strm>>>(A, part, span))
+#define NERVE_INT4_GEMV(GG)                                                                               \
+    (batch_width == 1 ? (zp ? NERVE_INT4_GEMV_FORM(GG, true, 1) : NERVE_INT4_GEMV_FORM(GG, false, 1))     \
+                      : (zp ? NERVE_INT4_GEMV_FORM(GG, true, 4) : NERVE_INT4_GEMV_FORM(GG, false, 4)))
             if (A.G == 128) NERVE_INT4_GEMV(128);
             else if (A.G == 64) NERVE_INT4_GEMV(64);
             else if (A.G == 32) NERVE_INT4_GEMV(32);
             else NERVE_INT4_GEMV(256);
 #undef NERVE_INT4_GEMV
+#undef NERVE_INT4_GEMV_FORM
             if (part) nh::int4_split_sum(A, part, splits, strm);
             return nh::check_launch("int4_linear_gptq_gemv");
         }
