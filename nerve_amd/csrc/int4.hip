@@ -588,7 +588,7 @@ __global__ __launch_bounds__(256) void int4_pp_kernel(PpArgs P) {
 // contracts exactly one 32-column activation block, so its int32 result is
 // the block's exact dot and each block is folded as acc_g = fma(dot, s_x,
 // acc_g), a segment of blocks that share a weight scale as acc = fma(acc_g,
-// s_w, acc).
+// s_w, acc), s_x times I8_SCALE_DOWN.
 //
 // A wave owns 16 J columns and 16 MT tokens and the block's KS waves split the
 // blocks of K.  Operands: lane (g = l / 16, r = l % 16) supplies 8 bytes of
@@ -679,7 +679,7 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
         for (int v = 0; v < NV; v++) {
             const uint32_t i = v * 64 + lane, t = min(m0 + i / U, M - 1), bb = b + i % U;
             const float s = P.s[(uint64_t)t * nblk + min(bb, b1 - 1)];
-            B.sx[v] = bb < b1 ? s : 0.0f;
+            B.sx[v] = bb < b1 ? s * I8_SCALE_DOWN : 0.0f;
         }
     };
     typedef float rows_t __attribute__((ext_vector_type(RT)));
@@ -779,6 +779,7 @@ __global__ __launch_bounds__(64 * KS) void int4_i8_kernel(PpArgs P, uint32_t tgr
             float v = part[0][c % J][l][t % RT];
 #pragma unroll
             for (int w = 1; w < KS; w++) v += part[w][c % J][l][t % RT];
+            v *= I8_SCALE_UP;
             if (split_part) split_part[((uint64_t)blockIdx.y * M + tt) * N + n0 + c] = v;
             else finalize_store(A, tt, n0 + c, v);
         }

@@ -73,6 +73,15 @@ __device__ __forceinline__ float load_scale(const uint16_t* p, bool bf16) { retu
 
 constexpr uint32_t ONES_BF16 = 0x3F803F80u;
 
+// The matrix-core forms for INT8 rows add a segment's dots times their activation
+// scales before the weight scale comes in.  A block's dot reaches 32 * 127 * 8 and
+// a segment has up to four blocks, so with bf16 rows near the type's limit (scales
+// up to 2^121) that sum passes the largest f32 although the result, fma(dot,
+// s_x s_w, sum) in the shader, does not.  The activation scales are therefore
+// taken 2^-11 times (130048 * 2^121 * 2^-11 < 2^128) and the sum 2^11 times at the
+// end; both are exact, so ordinary results keep every bit.
+constexpr float I8_SCALE_DOWN = 0x1p-11f, I8_SCALE_UP = 0x1p11f;
+
 __device__ __forceinline__ void finalize_store(const Int4Args& A, uint32_t t, uint32_t n, float sum) {
     // nerve/model_package_shader_selection.py:2504-2533
     float v = sum;

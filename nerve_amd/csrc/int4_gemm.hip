@@ -190,7 +190,7 @@ __global__ __launch_bounds__(GT_THREADS, 2) void int4_gemm_kernel(GemmArgs P) {
                 sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, false);   // lanes 2 b, 2 b + 1: block b
                 if ((p8 & 1) == 0) {
                     rsum[buf][(p8 >> 1) % NSUM][t] = (float)(-136 * sum);
-                    rsx[buf][p8 >> 1][t] = S.sx[i];
+                    rsx[buf][p8 >> 1][t] = S.sx[i] * I8_SCALE_DOWN;
                 }
             }
         }
@@ -331,6 +331,10 @@ __global__ __launch_bounds__(GT_THREADS, 2) void int4_gemm_kernel(GemmArgs P) {
         for (int i = 0; i < 4; i++) {
             const uint32_t t = m0 + 16 * m + 4 * g + i;
             if (t >= M) continue;
+            if (I8) {
+#pragma unroll
+                for (int j = 0; j < GJ; j++) acc[m][j][i] *= I8_SCALE_UP;
+            }
             if (P.part) {
                 float* p = P.part + ((uint64_t)split * M + t) * N;
                 if (CT) {

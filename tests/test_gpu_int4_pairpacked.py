@@ -226,3 +226,35 @@ def test_int4_linear_prequant_tiles(ctx, dev, kind, M, K, N, G):
                                      (48, 1344, 8320, 96), (47, 2048, 8256, 128)])
 def test_int4_linear_prequant_row_groups(ctx, dev, kind, M, K, N, G):
     test_int4_linear_prequant_tiles(ctx, dev, kind, M, K, N, G)
+
+
+# Rows near bf16's limit with results well inside it: a segment's dots times their
+# activation scales pass the largest f32 unless the kernels scale them down.  One
+# token per lane group, one and three token tiles, the tiled split-K form; segments
+# of four, two and one blocks.
+@pytest.mark.parametrize("kind", ["paired", "gptq", "ct"])
+@pytest.mark.parametrize("M,K,N,G", [(1, 512, 96, 128), (16, 1024, 8256, 64), (48, 1344, 8320, 96), (70, 512, 320, 128)])
+def test_int4_linear_prequant_large_rows(ctx, dev, kind, M, K, N, G):
+    import torch
+
+    rng = np.random.default_rng(M + K + N + G)
+    d = wl.int4_gptq(rng, K, N, G, True)
+    d["scales"] = wl.bf16_bits_to_f32(wl.f32_to_bf16_bits(d["scales"].astype(np.float32) * np.float32(2.0 ** -8)))
+    qw, sc = _ct_layout(d, K, N) if kind == "ct" else (d["qweight"], d["scales"])
+    sc_bits = wl.f32_to_bf16_bits(sc)
+    # standard normal times 2^125, held below the largest bf16
+    x = wl.f32_to_bf16_bits(np.clip(rng.standard_normal((M, K)), -7.9, 7.9).astype(np.float32) * np.float32(2.0 ** 125))
+    q, s, sums = _quant(ctx, dev, x) if kind == "paired" else (*_quant_unpaired(ctx, dev, x), None)
+    y = torch.zeros(M, N, dtype=torch.int16, device=dev)
+    spec = (f"linear_prequant{'_pairpacked' if kind == 'paired' else ''}_batch16_int4_{'ct' if kind == 'ct' else 'gptq'}"
+            f"_sbf16_g{G}_{K}x{N}.comp")
+    ctx.int4_linear_pairpacked(spec, q, s, sums, to_dev(qw, dev), to_dev(sc_bits, dev), None, y, M)
+    if kind == "paired":
+        qr, sr, sumr = oracle.quantize_i8_pairpacked(x)
+        ref = oracle.int4_linear_pairpacked(qr, sr, sumr, qw, sc_bits, G, scale_bf16=True)
+    else:
+        qr, sr = oracle.quantize_i8(x)
+        ref = oracle.int4_linear_prequant(kind, qr, sr, qw, sc_bits, G, scale_bf16=True)
+    assert np.all(np.isfinite(wl.bf16_bits_to_f32(ref)))
+    ok, worst, exact = bf16_close(to_np(y, np.uint16), ref, atol=linear_atol(x, gptq_dequant(d)), name="prequant large")
+    assert ok and exact > 0.9, (worst, exact)
