@@ -277,11 +277,20 @@ __global__ __launch_bounds__(64 * SM_WAVES) void sparse_int4_kernel(SmArgs A) {
 //
 // A block owns a window of `group` route positions and 16 NW output channels.
 // Positions of one expert that follow each other in the map form a run (the
-// compaction sorts the map, so an expert is one run; an owned range leaves the
-// map in source order and the runs are shorter), and every TS-th position of a
-// run starts a tile of up to TS routes.  The block takes the tiles that start
+// compaction sorts the map, so an expert is one run), and every TS-th position of
+// a run starts a tile of up to TS routes.  The block takes the tiles that start
 // in its window, so an expert's weights are decoded once per TS routes and not
 // once per route.
+//
+// An owned range leaves the map in source order, where runs are mostly one route
+// long, and fills only a part of it.  Its positions are dealt to all windows and a
+// run is then the expert's positions within SM_CHUNK, whose expert ids the block
+// stages in LDS where the tile's rows go afterwards (2 KB of their own cost
+// K = 4096 its third block a CU: 16 tokens over 128 experts top 8 174 us against
+// 163).  The routed block at h3072 i1024 e256 k10, us with a block per route /
+// runs of neighbours in windows of the whole map / this: 32 owned experts and 103
+// tokens 278 / 271 / 114, 128 and 256 1585 / 1847 / 635, 256 and 1024
+// 10665 / 12618 / 5360.
 //
 // A wave owns 16 channels: 16 weight rows of gate and the same of up (down: 32
 // rows).  Panels of PANEL columns of these rows stream through registers two
@@ -311,8 +320,11 @@ __device__ __forceinline__ uint32_t sm_pair_exponent() {   // see pair_exponent(
     return e;
 }
 
+constexpr uint32_t SM_CHUNK = 1024;
+
 // LDS rows are padded by 16 bytes: 16 rows' operand reads hit distinct banks
 // at immediate offsets.  LDS bytes of one block:
+constexpr uint32_t TILE_LDS_MOST = 160 * 1024 - 256;     // beside the static tables
 constexpr uint32_t tile_lds(uint32_t K, uint32_t TS, uint32_t NW, uint32_t PANEL) {
     return TS * (K * 2 + 16) + NW * 2 * 16 * (PANEL / 2 + 16 + PANEL / 16);
 }
@@ -356,32 +368,68 @@ __global__ __launch_bounds__(64 * NW, WPE) void sparse_tile_kernel(SmArgs A, uin
         const uint32_t e = word & 0xffffu;
         return (e >= A.E || (count != 0u && (e < start || e - start >= count))) ? 0xffffffffu : e;
     };
-    for (uint32_t p = win * group; p < min(npos, (win + 1) * group); p++) {
-        // ---- the tile at position p, by every wave for itself: lane l looks
-        // at position p + l (the tile's routes) and p - 1 - l (the run's start).
-        uint32_t c, word, cb, wb;
-        const uint32_t ef = route_at(p + lane, c, word);
-        uint32_t eb = route_at(lane < p ? p - 1 - lane : 0xffffffffu, cb, wb);
-        const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)ef);
-        if (e == 0xffffffffu) continue;
-        uint32_t back = 0;                                              // positions of the run before p
-        for (;;) {
-            const uint64_t other = __ballot(eb != e);
-            if (other) {
-                back += (uint32_t)__builtin_ctzll(other);
-                break;
+    // Owned: windows take every A.npos-th position, since the first positions of a
+    // chunk hold most of its tiles.
+    const bool owned = count != 0u;
+    const uint32_t step = owned ? A.npos : 1u, last = owned ? npos : min(npos, (win + 1) * group);
+    uint16_t* chunk_e = reinterpret_cast<uint16_t*>(lds);               // owned: experts of the chunk's positions
+    uint32_t staged = 0xffffffffu;                                      // first position of the chunk in LDS
+    for (uint32_t p = owned ? win : win * group; p < last; p += step) {
+        // ---- the tile at position p, by every wave for itself.
+        const uint32_t c0 = p / SM_CHUNK * SM_CHUNK, c1 = min(npos, c0 + SM_CHUNK);
+        uint32_t e, back = 0, nt = 0, c = 0, word = 0;                  // back: positions of the run before p
+        if (owned) {
+            if (staged != c0) {
+                __syncthreads();                                        // the previous tile's reads are done
+                for (uint32_t i = c0 + tid; i < c1; i += 64 * NW) chunk_e[i - c0] = (uint16_t)route_at(i, c, word);
+                __syncthreads();
+                staged = c0;
             }
-            back += 64;
-            eb = route_at(back + lane < p ? p - 1 - back - lane : 0xffffffffu, cb, wb);
+            e = (uint32_t)__builtin_amdgcn_readfirstlane((int)chunk_e[p - c0]);
+            if (e == 0xffffu) continue;
+            for (uint32_t i = c0; i < p; i += 64)
+                back += (uint32_t)__popcll(__ballot(i + lane < p && chunk_e[i + lane - c0] == e));
+            if (back % TS) continue;
+        } else {
+            // Lane l looks at position p + l (the tile's routes) and p - 1 - l (the
+            // run's start).
+            uint32_t cb, wb;
+            const uint32_t ef = route_at(p + lane, c, word);
+            uint32_t eb = route_at(lane < p ? p - 1 - lane : 0xffffffffu, cb, wb);
+            e = (uint32_t)__builtin_amdgcn_readfirstlane((int)ef);
+            if (e == 0xffffffffu) continue;
+            for (;;) {
+                const uint64_t other = __ballot(eb != e);
+                if (other) {
+                    back += (uint32_t)__builtin_ctzll(other);
+                    break;
+                }
+                back += 64;
+                eb = route_at(back + lane < p ? p - 1 - back - lane : 0xffffffffu, cb, wb);
+            }
+            if (back % TS) continue;
+            const uint64_t fend = __ballot(ef != e);
+            nt = min(TS, fend ? (uint32_t)__builtin_ctzll(fend) : 64u);
         }
-        if (back % TS) continue;
-        const uint64_t fend = __ballot(ef != e);
-        const uint32_t nt = min(TS, fend ? (uint32_t)__builtin_ctzll(fend) : 64u);
         const uint32_t* W = static_cast<const uint32_t*>(sm_param(A, 2 * e, A.w_bytes, 16));
         const uint16_t* S = static_cast<const uint16_t*>(sm_param(A, 2 * e + 1, A.s_bytes, 2));
         if (!W || !S) continue;                                         // uniform over the block
         __syncthreads();                                                // the previous tile's reads are done
-        if (tid < TS) {
+        if (owned) {
+            for (uint32_t i = p; i < c1 && nt < TS; i += 64) {
+                const bool mine = i + lane < c1 && chunk_e[i + lane - c0] == e;
+                const uint64_t m = __ballot(mine);
+                const uint32_t t = nt + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+                if (wave == 0 && mine && t < TS) {
+                    route_at(i + lane, c, word);
+                    t_route[t] = c;
+                    t_word[t] = word;
+                }
+                nt += (uint32_t)__popcll(m);
+            }
+            nt = min(TS, nt);
+            staged = 0xffffffffu;                                       // the rows overwrite the ids
+        } else if (tid < TS) {
             t_route[tid] = c;
             t_word[tid] = word;
         }
@@ -511,7 +559,7 @@ nerve_hip_status launch_tile_form(SmArgs A, uint32_t group, hipStream_t stream) 
     auto* kernel = A.scale_bf16 ? sparse_tile_kernel<GATE_UP, TS, NW, PANEL, WPE, true> : sparse_tile_kernel<GATE_UP, TS, NW, PANEL, WPE, false>;
     static bool attr_set[2] = {false, false};
     if (!attr_set[A.scale_bf16 ? 1 : 0]) {
-        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256) != hipSuccess)
+        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, TILE_LDS_MOST) != hipSuccess)
             return nh::fail(NERVE_HIP_DEVICE_ERROR, "hipFuncSetAttribute failed for sparse_tile_kernel");
         attr_set[A.scale_bf16 ? 1 : 0] = true;
     }
@@ -522,7 +570,6 @@ nerve_hip_status launch_tile_form(SmArgs A, uint32_t group, hipStream_t stream) 
 // The tile form, or UNSUPPORTED where its loads or its LDS do not fit.
 template <bool GATE_UP>
 nerve_hip_status launch_tiles(const SmArgs& A, hipStream_t stream) {
-    constexpr uint32_t MOST = 160 * 1024 - 256;
     if (A.G % 32 || (A.G & (A.G - 1)) || A.K % 128 || A.N % 16) return NERVE_HIP_UNSUPPORTED;
     // Routes per expert if they spread evenly: a tile takes 4, 8 or 16 routes,
     // since its rows in LDS (2 K bytes each) cost blocks per CU.  The routed
@@ -531,9 +578,9 @@ nerve_hip_status launch_tiles(const SmArgs& A, hipStream_t stream) {
     // 8 positions where most of them start no tile.
     const uint32_t per = A.npos / A.E;
     const uint32_t group = per >= 4 ? 8 : 1;
-    if (per < 3 && tile_lds(A.K, 4, 4, 256) <= MOST) return launch_tile_form<GATE_UP, 4, 4, 256, 3>(A, group, stream);
-    if (per < 8 && tile_lds(A.K, 8, 4, 256) <= MOST) return launch_tile_form<GATE_UP, 8, 4, 256, 2>(A, group, stream);
-    if (tile_lds(A.K, 16, 8, 256) <= MOST) return launch_tile_form<GATE_UP, 16, 8, 256, 2>(A, group, stream);
+    if (per < 3 && tile_lds(A.K, 4, 4, 256) <= TILE_LDS_MOST) return launch_tile_form<GATE_UP, 4, 4, 256, 3>(A, group, stream);
+    if (per < 8 && tile_lds(A.K, 8, 4, 256) <= TILE_LDS_MOST) return launch_tile_form<GATE_UP, 8, 4, 256, 2>(A, group, stream);
+    if (tile_lds(A.K, 16, 8, 256) <= TILE_LDS_MOST) return launch_tile_form<GATE_UP, 16, 8, 256, 2>(A, group, stream);
     return NERVE_HIP_UNSUPPORTED;
 }
 

@@ -144,8 +144,9 @@ def test_batched_shapes(ctx, dev, H, I, G, sbf, B):
 # expert), runs cut at a tile and longer than a wave (the run's start is then
 # searched over several rounds), windows of one and eight positions, one panel,
 # a panel and a half and an odd number of them, output rows cut at a block's
-# channels, f16 and bf16 scales of one and several blocks, and an owned range
-# (runs of a map in source order).
+# channels, f16 and bf16 scales of one and several blocks, and owned ranges (a map
+# in source order, whose tiles gather an expert's positions: every tile size, a map
+# of one position, windows of several positions, more than one chunk of 1024).
 @pytest.mark.parametrize("H,I,G,sbf,E,k,B,owned", [
     (128, 128, 32, True, 8, 2, 5, None),
     (384, 640, 32, False, 16, 3, 20, None),
@@ -153,6 +154,12 @@ def test_batched_shapes(ctx, dev, H, I, G, sbf, B):
     (256, 384, 128, False, 3, 2, 70, None),
     (512, 256, 32, True, 2, 1, 300, None),
     (384, 128, 32, True, 6, 3, 50, (2, 3)),
+    (256, 128, 32, True, 64, 2, 1, (0, 63)),
+    (128, 256, 64, False, 64, 2, 40, (8, 48)),
+    (256, 128, 32, False, 16, 3, 20, (3, 12)),
+    (128, 128, 32, True, 16, 4, 30, (0, 16)),
+    (128, 128, 32, True, 8, 2, 700, (1, 6)),
+    (128, 128, 32, True, 24, 2, 1100, (0, 24)),
 ])
 def test_tile_form(ctx, dev, H, I, G, sbf, E, k, B, owned):
     rig = Rig(dev, H, I, E, k, G, sbf, nb=E, seed=H + I + B)
