@@ -567,26 +567,51 @@ nerve_hip_status launch_tile_form(SmArgs A, uint32_t group, hipStream_t stream) 
     return nh::check_launch(GATE_UP ? "int4_moe_gate_up" : "int4_moe_down");
 }
 
-// The tile form, or UNSUPPORTED where its loads or its LDS do not fit.
+// The tile form, or UNSUPPORTED where its loads do not fit or where a block per
+// route is the faster one.
 template <bool GATE_UP>
-nerve_hip_status launch_tiles(const SmArgs& A, hipStream_t stream) {
+nerve_hip_status launch_tiles(const SmArgs& A, uint32_t cus, hipStream_t stream) {
     if (A.G % 32 || (A.G & (A.G - 1)) || A.K % 128 || A.N % 16) return NERVE_HIP_UNSUPPORTED;
-    // Routes per expert if they spread evenly: a tile takes 4, 8 or 16 routes,
-    // since its rows in LDS (2 K bytes each) cost blocks per CU.  The routed
-    // block at h3072 i1024 e256 k10, us by tile size 4 / 8 / 16 at 16, 64 and
-    // 256 tokens: 180 / 191 / 219, 396 / 403 / 457, 976 / 740 / 594.  Windows of
-    // 8 positions where most of them start no tile.
+    // Few blocks: a tile's chain (route, record, rows, panels two ahead) is longer
+    // than that of the kernel per route, which has all of its weights in flight at
+    // once, and only several rounds of blocks hide it.  One token, gate_up, us by
+    // tile / by route: h3072 i1024 top 10 20.4 / 15.1, h2048 i768 top 4 13.9 / 6.8;
+    // from 8 blocks a CU on: 160 routes of h3072 i1024 93.8 / 115.4, 96 of h2048
+    // i1408 48.3 / 59.1.
+    const uint64_t rows = GATE_UP ? 64 : 128;
+    if ((uint64_t)A.npos * ((A.N + rows - 1) / rows) < 8ull * cus) return NERVE_HIP_UNSUPPORTED;
+    // Routes per expert if they spread evenly.  Groups longer than 32 take their
+    // scales two bytes a load and need two (60 experts, h2048 i1408 g64, 64 routes
+    // 53.5 / 42.3, 128 routes 73.4 / 76.6).
     const uint32_t per = A.npos / A.E;
+    if (A.G != 32 && per < 2) return NERVE_HIP_UNSUPPORTED;
+    // A tile takes 4, 8 or 16 routes: its rows in LDS (2 K bytes each) cost blocks
+    // per CU.  The routed block at h3072 i1024 e256 k10, us by tile size 4 / 8 / 16
+    // at 16, 64 and 256 tokens: 180 / 191 / 219, 396 / 403 / 457, 976 / 740 / 594.
+    // Blocks of four waves need a second one on the CU (gate_up of 128 routes of 16
+    // experts, K = 4096, by 4 / 8 / route: 484 / 581 / 1048 us; down of 64 routes of
+    // 8, K = 14336, 403 by 4, 282 by route), or 8 routes from four per expert on
+    // (128 routes of 32, K = 8192: 460 / 731).
+    const uint32_t lds4 = tile_lds(A.K, 4, 4, 256), lds8 = tile_lds(A.K, 8, 4, 256), lds16 = tile_lds(A.K, 16, 8, 256);
+    constexpr uint32_t LDS = 160 * 1024;
+    uint32_t ts = per < 3 ? 4 : per < 8 ? 8 : 16;
+    if (ts == 16 && lds16 > TILE_LDS_MOST) ts = 8;
+    if (2 * lds4 > LDS) {
+        if (per < 4 || lds8 > TILE_LDS_MOST) return NERVE_HIP_UNSUPPORTED;
+        ts = 8;
+    } else if (ts == 8 && 2 * lds8 > LDS) {
+        ts = 4;
+    }
+    // Windows of 8 positions where most of them start no tile.
     const uint32_t group = per >= 4 ? 8 : 1;
-    if (per < 3 && tile_lds(A.K, 4, 4, 256) <= TILE_LDS_MOST) return launch_tile_form<GATE_UP, 4, 4, 256, 3>(A, group, stream);
-    if (per < 8 && tile_lds(A.K, 8, 4, 256) <= TILE_LDS_MOST) return launch_tile_form<GATE_UP, 8, 4, 256, 2>(A, group, stream);
-    if (tile_lds(A.K, 16, 8, 256) <= TILE_LDS_MOST) return launch_tile_form<GATE_UP, 16, 8, 256, 2>(A, group, stream);
-    return NERVE_HIP_UNSUPPORTED;
+    if (ts == 4) return launch_tile_form<GATE_UP, 4, 4, 256, 3>(A, group, stream);
+    if (ts == 8) return launch_tile_form<GATE_UP, 8, 4, 256, 2>(A, group, stream);
+    return launch_tile_form<GATE_UP, 16, 8, 256, 2>(A, group, stream);
 }
 
 template <bool GATE_UP>
-nerve_hip_status launch_sparse(const SmArgs& A, hipStream_t stream) {
-    const nerve_hip_status tiled = launch_tiles<GATE_UP>(A, stream);
+nerve_hip_status launch_sparse(const SmArgs& A, uint32_t cus, hipStream_t stream) {
+    const nerve_hip_status tiled = launch_tiles<GATE_UP>(A, cus, stream);
     if (tiled != NERVE_HIP_UNSUPPORTED) return tiled;
     const uint32_t units = A.K / 32;
     const bool spw = A.G % 32 != 0;
@@ -658,7 +683,8 @@ nerve_hip_status sparse_common(nerve_hip_ctx* ctx, const char* spec, bool gate_u
     A.s_bytes = wrows * (K / ms.group) * 2;
     A.batched = ms.batch1 ? 1 : 0;
     A.scale_bf16 = ms.scale_bf16;
-    return gate_up ? launch_sparse<true>(A, (hipStream_t)stream) : launch_sparse<false>(A, (hipStream_t)stream);
+    const uint32_t cus = (uint32_t)ctx->cu_count;
+    return gate_up ? launch_sparse<true>(A, cus, (hipStream_t)stream) : launch_sparse<false>(A, cus, (hipStream_t)stream);
 }
 
 }  // namespace

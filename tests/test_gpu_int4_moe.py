@@ -140,13 +140,9 @@ def test_batched_shapes(ctx, dev, H, I, G, sbf, B):
     _check(rig, x, routes, h, y)
 
 
-# The matrix-core tile form: every tile size (4, 8, 16 routes, by routes per
-# expert), runs cut at a tile and longer than a wave (the run's start is then
-# searched over several rounds), windows of one and eight positions, one panel,
-# a panel and a half and an odd number of them, output rows cut at a block's
-# channels, f16 and bf16 scales of one and several blocks, and owned ranges (a map
-# in source order, whose tiles gather an expert's positions: every tile size, a map
-# of one position, windows of several positions, more than one chunk of 1024).
+# Shapes that the tile form's loads take, with too few blocks for it: the kernel per
+# route over experts with many routes, f16 and bf16 scales of one and several
+# blocks, and owned ranges (a map in source order).
 @pytest.mark.parametrize("H,I,G,sbf,E,k,B,owned", [
     (128, 128, 32, True, 8, 2, 5, None),
     (384, 640, 32, False, 16, 3, 20, None),
@@ -163,6 +159,37 @@ def test_batched_shapes(ctx, dev, H, I, G, sbf, B):
 ])
 def test_tile_form(ctx, dev, H, I, G, sbf, E, k, B, owned):
     rig = Rig(dev, H, I, E, k, G, sbf, nb=E, seed=H + I + B)
+    routes, _ = oracle.topk(wl.bf16_normal(rig.rng, (B, E)), k, telemetry=False)
+    routes = routes.astype(np.uint32)
+    x = wl.bf16_normal(rig.rng, (B, H))
+    start, count = owned or (0, 0)
+    h, y, _, _ = _run_batched(ctx, rig, x, routes, B, start, count)
+    _check(rig, x, routes, h, y, start, count)
+
+
+# The matrix-core tile form (from 8 blocks a CU on: here 2048 routes or 128-row
+# tiles): every tile size (4, 8, 16 routes, by routes per expert and by the LDS of
+# its rows: K = 4096 takes 4 and K = 8192 takes 8 where shorter rows take 16), runs cut
+# at a tile and longer than a wave (the run's start is then searched over several
+# rounds), windows of one and eight positions, one panel, a panel and a half and an
+# odd number of them, output rows cut at a block's channels, f16 and bf16 scales of one
+# and several blocks, and owned ranges (a map in source order, whose tiles gather an
+# expert's positions within a chunk of 1024).
+@pytest.mark.parametrize("H,I,G,sbf,E,k,B,owned", [
+    (128, 128, 32, True, 1024, 2, 1030, None),
+    (384, 640, 32, False, 400, 2, 1100, None),
+    (640, 128, 64, True, 100, 2, 1030, None),
+    (256, 384, 128, False, 64, 3, 700, None),
+    (384, 128, 32, True, 2, 1, 2100, None),
+    (4096, 256, 32, True, 16, 2, 300, None),
+    (8192, 256, 32, False, 64, 2, 300, None),
+    (128, 256, 32, True, 1024, 2, 1030, (100, 700)),
+    (256, 128, 32, False, 400, 2, 1100, (0, 399)),
+    (256, 128, 32, True, 400, 2, 1100, (7, 9)),
+    (128, 128, 64, True, 64, 2, 1100, (3, 40)),
+])
+def test_tile_form_many_routes(ctx, dev, H, I, G, sbf, E, k, B, owned):
+    rig = Rig(dev, H, I, E, k, G, sbf, nb=min(E, 8), seed=H + I + B + E)
     routes, _ = oracle.topk(wl.bf16_normal(rig.rng, (B, E)), k, telemetry=False)
     routes = routes.astype(np.uint32)
     x = wl.bf16_normal(rig.rng, (B, H))
