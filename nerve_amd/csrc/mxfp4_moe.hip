@@ -1527,8 +1527,11 @@ __device__ __forceinline__ uint32_t sload_u32(const uint32_t* p) {
 // that split each item's K chunks.  An item is RI = 16 NSUB rows of each of
 // the NMAT matrices.
 // QIN: the activation rows are e4m3 with pow2 block scales (A.aq, A.as); bf16
-// rows (A.x16) are quantized in registers otherwise.
-template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool QIN>
+// rows (A.x16) are quantized in registers otherwise.  PAD: LDS rows have a gap
+// (A.w_stride != K / 2).  Its offsets take registers: down at K = 2880, which needs
+// no gap, spills 14 with PAD false and 17 with it (a layer of one token over 32
+// experts 37.55 us against 37.85; 37.3 before rows had gaps).
+template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool QIN, bool PAD>
 __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, uint32_t i1, uint32_t nrb,
                                              const TileSrc& ts) {
     constexpr uint32_t RI = 16 * NSUB;
@@ -1576,10 +1579,14 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
 #pragma unroll
     for (uint32_t t = 0; t < LWMAX; t++)
         wsrc[t] = A.block_major ? ((woff[t] % RB) / 64) * N * 64 + (woff[t] / RB) * 64 + woff[t] % 64 : woff[t];
-    // LDS offsets: rows A.w_stride apart (a 16-byte piece never straddles a row).
-    uint32_t wdst[LWMAX];
+    // LDS offsets: rows WS apart (a 16-byte piece never straddles a row).
+    const uint32_t WS = PAD ? A.w_stride : RB;
+    uint32_t wpad[PAD ? LWMAX : 1];
+    if constexpr (PAD) {
 #pragma unroll
-    for (uint32_t t = 0; t < LWMAX; t++) wdst[t] = woff[t] + __umulhi(woff[t], A.row_magic) * (A.w_stride - RB);
+        for (uint32_t t = 0; t < LWMAX; t++) wpad[t] = woff[t] + __umulhi(woff[t], A.row_magic) * (WS - RB);
+    }
+    auto wdst = [&](uint32_t t) __attribute__((always_inline)) { return PAD ? wpad[PAD ? t : 0] : woff[t]; };
 #pragma unroll
     for (uint32_t t = 0; t < LSMAX; t++)
         ssrc[t] = A.block_major ? ((soff[t] % SB) / 4) * N * 4 + (soff[t] / SB) * 4 : soff[t];
@@ -1616,7 +1623,7 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
         for (int m = 0; m < NMAT; m++) {
 #pragma unroll
             for (uint32_t t = 0; t < LWMAX; t++)
-                if (t < lw) *reinterpret_cast<v4i*>(dst + m * A.w_region + wdst[t]) = R.w[m][t];
+                if (t < lw) *reinterpret_cast<v4i*>(dst + m * A.w_region + wdst(t)) = R.w[m][t];
 #pragma unroll
             for (uint32_t t = 0; t < LSMAX; t++)
                 if (t < ls) *reinterpret_cast<uint32_t*>(dst + NMAT * A.w_region + m * A.s_region + soff[t]) = R.s[m][t];
@@ -1633,7 +1640,7 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
         const uint32_t c = c0 + q, kb = c * 128 + g * 32;
         kvalid[q] = c < c1 && kb < K;
         const uint32_t kk = kvalid[q] ? kb : 0;
-        rw[q] = rr * A.w_stride + kk / 2;
+        rw[q] = rr * WS + kk / 2;
         rs[q] = NMAT * A.w_region + rr * SB + kk / 32;
     }
 
@@ -1780,7 +1787,7 @@ __device__ __forceinline__ void stream_range(const StreamArgs& A, uint32_t i0, u
                 for (int m = 0; m < NMAT; m++) {
 #pragma unroll
                     for (int j = 0; j < NSUB; j++) {
-                        w[u][m][j] = lds_read16(buf + m * A.w_region + j * 16 * A.w_stride + rw[q0 + u]);
+                        w[u][m][j] = lds_read16(buf + m * A.w_region + j * 16 * WS + rw[q0 + u]);
                         sw[u][m][j] = lds_read_u8(buf + m * A.s_region + j * 16 * SB + rs[q0 + u]);
                     }
                 }
@@ -2207,7 +2214,7 @@ __device__ __forceinline__ void fused_small_plan(const TileArgs& A, SmallPlan& S
     __syncthreads();
 }
 
-template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool FUSED, bool QIN>
+template <int MODE, int NMAT, int NBUF, int NW, int NSUB, bool FUSED, bool QIN, bool PAD>
 __global__ __launch_bounds__(64 * NW) void mx_stream_kernel(StreamArgs A) {
     extern __shared__ __attribute__((aligned(16))) uint8_t ring[];
     if (A.count_control && blockIdx.x == 0 && threadIdx.x == 0) {
@@ -2237,7 +2244,7 @@ __global__ __launch_bounds__(64 * NW) void mx_stream_kernel(StreamArgs A) {
         ts.out_route = ov ? S.route[tl] : 0u;
         ts.out_word = ov ? S.word[tl] : 0u;
         lds_drain();   // the plan is read before any copy can overwrite it
-        stream_range<MODE, NMAT, NBUF, NW, NSUB, QIN>(A, tile * nrb + lo_rb, tile * nrb + hi_rb, nrb, ts);
+        stream_range<MODE, NMAT, NBUF, NW, NSUB, QIN, PAD>(A, tile * nrb + lo_rb, tile * nrb + hi_rb, nrb, ts);
         return;
     }
     if (FUSED) {
@@ -2278,13 +2285,13 @@ __global__ __launch_bounds__(64 * NW) void mx_stream_kernel(StreamArgs A) {
         block_share(G, b, n_tiles, nrb, tile, lo_rb, hi_rb);
         if (lo_rb >= hi_rb) return;
         const TileSrc ts = tile_src(tile);
-        stream_range<MODE, NMAT, NBUF, NW, NSUB, QIN>(A, tile * nrb + lo_rb, tile * nrb + hi_rb, nrb, ts);
+        stream_range<MODE, NMAT, NBUF, NW, NSUB, QIN, PAD>(A, tile * nrb + lo_rb, tile * nrb + hi_rb, nrb, ts);
     } else {
         for (uint32_t t = b; t < n_tiles; t += G) {
             // The tables share LDS with the ring: rebuild them after a range.
             if (FUSED && t != b) fused_tables<NW>(A.T, F, addr_lds);
             const TileSrc ts = tile_src(t);
-            stream_range<MODE, NMAT, NBUF, NW, NSUB, QIN>(A, t * nrb, (t + 1) * nrb, nrb, ts);
+            stream_range<MODE, NMAT, NBUF, NW, NSUB, QIN, PAD>(A, t * nrb, (t + 1) * nrb, nrb, ts);
         }
     }
 }
@@ -2328,14 +2335,20 @@ nerve_hip_status launch_stream(StreamArgs A, const nerve_hip_ctx* ctx, hipStream
             ((uintptr_t)A.T.addr & 15))
             return NERVE_HIP_UNSUPPORTED;
     }
-    static bool attr_set = false;
-    if (!attr_set) {
-        if (hipFuncSetAttribute((const void*)mx_stream_kernel<MODE, NMAT, NBUF, NW, NSUB, FUSED, QIN>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
+    // The gate/up form on e4m3 rows keeps the gap's registers for every K: without
+    // them it is scheduled worse (K = 2880, 128 experts, 16 / 64 tokens 144.5 / 314 us
+    // a layer against 143.6 / 310.5).
+    constexpr bool ALWAYS = MODE == SPAN_GATE_UP && QIN;
+    const bool pad = ALWAYS || A.w_stride != A.K / 2;
+    auto* kernel = pad ? mx_stream_kernel<MODE, NMAT, NBUF, NW, NSUB, FUSED, QIN, true>
+                       : mx_stream_kernel<MODE, NMAT, NBUF, NW, NSUB, FUSED, QIN, ALWAYS>;
+    static bool attr_set[2] = {false, false};
+    if (!attr_set[pad]) {
+        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024) != hipSuccess)
             return nh::fail(NERVE_HIP_DEVICE_ERROR, "hipFuncSetAttribute failed for mx_stream_kernel");
-        attr_set = true;
+        attr_set[pad] = true;
     }
-    mx_stream_kernel<MODE, NMAT, NBUF, NW, NSUB, FUSED, QIN><<<ctx->cu_count, 64 * NW, lds, st>>>(A);
+    kernel<<<ctx->cu_count, 64 * NW, lds, st>>>(A);
     return nh::check_launch("mx_stream_kernel");
 }
 
@@ -2368,7 +2381,7 @@ constexpr uint32_t TOK_MAX_RECORDS = 512;            // address table staged by 
 
 // The body is a device function: the host pass instantiates kernel template
 // bodies, and the gfx950-only builtins below would fail there.
-template <int NBUF, int NW>
+template <int NBUF, int NW, bool PAD>
 __device__ __forceinline__ void mx_tokens_body(const StreamArgs& A) {
     constexpr uint32_t RI = 16, NMAT = 2, NSUB = 1;
     constexpr uint32_t CH = 24 / NW;                              // chunks per wave (K <= NW CH 128)
@@ -2578,9 +2591,13 @@ __device__ __forceinline__ void mx_tokens_body(const StreamArgs& A) {
         spos[q] = min(pc * 256, RI * SB - 256);
         soff[q] = spos[q] + lane * 4;
     }
-    uint32_t wdst[LWMAX];                     // LDS offsets: rows A.w_stride apart
+    const uint32_t WS = PAD ? A.w_stride : RB;   // LDS offsets: rows WS apart
+    uint32_t wpad[PAD ? LWMAX : 1];
+    if constexpr (PAD) {
 #pragma unroll
-    for (uint32_t q = 0; q < LWMAX; q++) wdst[q] = woff[q] + __umulhi(woff[q], A.row_magic) * (A.w_stride - RB);
+        for (uint32_t q = 0; q < LWMAX; q++) wpad[q] = woff[q] + __umulhi(woff[q], A.row_magic) * (WS - RB);
+    }
+    auto wdst = [&](uint32_t q) __attribute__((always_inline)) { return PAD ? wpad[PAD ? q : 0] : woff[q]; };
     // Item i: expert index i / nrb (u0 or u0 + 1), rows (i % nrb) * 16.
     // Its weight and scale bytes are loaded with nontemporal loads into a
     // register set (the same 1 KB / 256 B pieces per wave as a ring slot's
@@ -2614,7 +2631,7 @@ __device__ __forceinline__ void mx_tokens_body(const StreamArgs& A) {
         for (uint32_t m = 0; m < NMAT; m++) {
 #pragma unroll
             for (uint32_t q = 0; q < LWMAX; q++)
-                if (q < lw) *reinterpret_cast<v4i*>(dst + m * A.w_region + wdst[q]) = R.w[m][q];
+                if (q < lw) *reinterpret_cast<v4i*>(dst + m * A.w_region + wdst(q)) = R.w[m][q];
 #pragma unroll
             for (uint32_t q = 0; q < LSMAX; q++)
                 if (q < ls) *reinterpret_cast<uint32_t*>(dst + NMAT * A.w_region + m * A.s_region + soff[q]) = R.s[m][q];
@@ -2627,7 +2644,7 @@ __device__ __forceinline__ void mx_tokens_body(const StreamArgs& A) {
         const uint32_t c = c0 + q, kb = c * 128 + g * 32;
         kvalid[q] = c < c1 && kb < K;
         const uint32_t kk = kvalid[q] ? kb : 0;
-        rw[q] = rr * A.w_stride + kk / 2;
+        rw[q] = rr * WS + kk / 2;
         rs[q] = NMAT * A.w_region + rr * SB + kk / 32;
     }
 
@@ -2773,9 +2790,9 @@ __device__ __forceinline__ void mx_tokens_body(const StreamArgs& A) {
     }
 }
 
-template <int NBUF, int NW>
+template <int NBUF, int NW, bool PAD>
 __global__ __launch_bounds__(64 * NW) void mx_tokens_kernel(StreamArgs A) {
-    mx_tokens_body<NBUF, NW>(A);
+    mx_tokens_body<NBUF, NW, PAD>(A);
 }
 
 // Launches the token-form gate/up kernel, or returns UNSUPPORTED when the
@@ -2801,14 +2818,15 @@ nerve_hip_status launch_tokens(StreamArgs A, const nerve_hip_ctx* ctx, hipStream
     const size_t lds = (size_t)2 * A.slot_bytes + (size_t)NW * 2 * 64 * 16;
     const size_t plan = (sizeof(TokPlan) + 15) / 16 * 16 + (A.T.n_records > TOK_MAX_RECORDS ? 0 : (size_t)A.T.n_records * 32);
     if (lds > 160 * 1024 || plan > lds || A.copies_per_item * 2 > 63) return NERVE_HIP_UNSUPPORTED;
-    static bool attr_set = false;
-    if (!attr_set) {
-        if (hipFuncSetAttribute((const void*)mx_tokens_kernel<NBUF, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    auto* kernel = A.w_stride != A.K / 2 ? mx_tokens_kernel<NBUF, NW, true> : mx_tokens_kernel<NBUF, NW, false>;
+    static bool attr_set[2] = {false, false};
+    if (!attr_set[A.w_stride != A.K / 2]) {
+        if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 160 * 1024) != hipSuccess)
             return nh::fail(NERVE_HIP_DEVICE_ERROR, "hipFuncSetAttribute failed for mx_tokens_kernel");
-        attr_set = true;
+        attr_set[A.w_stride != A.K / 2] = true;
     }
-    mx_tokens_kernel<NBUF, NW><<<ctx->cu_count, 64 * NW, lds, st>>>(A);
+    kernel<<<ctx->cu_count, 64 * NW, lds, st>>>(A);
     return nh::check_launch("mx_tokens_kernel");
 }
 
