@@ -910,9 +910,15 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
             ((uintptr_t)scales & 7) == 0) {
             // Few column tiles and more than one batch per wave: K is split so
             // that every CU has a block, the partial sums added by a second
-            // launch (14336 x 4096, one row: 64 blocks 14.9 us, 256 10.1).
-            const uint32_t batches = (A.K / 8 + GEMV_ROWS - 1) / GEMV_ROWS;
-            const uint32_t most = std::max(1u, std::min((A.K / 256 + 15) / 16, (uint32_t)ctx->cu_count / tiles));
+            // launch (14336 x 4096, one row: 64 blocks 14.9 us, 256 10.1).  One row
+            // gains less: from K > 6144 on (unsplit / split, 4608 x 4096 7.2 / 7.9,
+            // 6144 x 8192 9.9 / 10.1, 7168 x 4096 9.9 / 9.2), later where half of the
+            // CUs have a tile (9216 x 6144 13.0 / 12.2, but 9216 x 8192 13.3 / 14.2,
+            // 11008 x 8192 15.7 / 15.3); two rows of 4608 x 4096 9.0 / 8.9, four
+            // 9.3 / 9.0.
+            const uint32_t batches = (A.K / 8 + GEMV_ROWS - 1) / GEMV_ROWS, cus = (uint32_t)ctx->cu_count;
+            const bool gains = batch_width > 1 || A.K > (2 * tiles >= cus ? 10240u : 6144u);
+            const uint32_t most = gains ? std::max(1u, std::min((A.K / 256 + 15) / 16, cus / tiles)) : 1u;
             const uint32_t span = (batches + most - 1) / most, splits = (batches + span - 1) / span;
             float* part = splits > 1 ? static_cast<float*>(ctx->split) : nullptr;
             dim3 g1((tiles + 7) / 8 * 8, splits);
