@@ -885,13 +885,34 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
     hipStream_t strm = (hipStream_t)stream;
     // More than 16 rows: the tiled split-K form, which expands the weights once per
     // 64 rows instead of once per 16; from five rows on also where column tiles are
-    // few and K is long (16 rows of 14336 x 4096: 25.4 -> 14.6 us).  The 16-row kernels stay where one
-    // round of their blocks covers a GPTQ linear with a short K (64 rows of
-    // 4096 x 4096: 10.1 against 15.1 us; of 14336 x 4096: 25.9 against 20.0).
-    const bool one_round = s.layout == 0 && A.N % 64 == 0 && A.K <= 6144 &&
-                           (uint64_t)(A.N / 64) * ((batch_width + 15) / 16) <= (uint64_t)ctx->cu_count;
-    const bool few = s.layout == 0 && A.N % 64 == 0 && batch_width > GEMV_MAX_M && A.K > 6144 &&
-                     2 * (A.N / 64) <= (uint32_t)ctx->cu_count;
+    // few and K is long (16 rows of 14336 x 4096: 25.4 -> 14.6 us).  The 16-row
+    // kernels stay where one round of their blocks covers the linear and K is short
+    // enough for the launch that adds the split sums to count (us, 16-row kernel /
+    // tiled form).
+    const uint32_t cus = (uint32_t)ctx->cu_count;
+    const uint64_t row_tiles16 = (batch_width + 15) / 16;
+    bool one_round = false;
+    if (s.layout == 0 && A.N % 64 == 0) {
+        // A block a CU: 64 rows of 4096 x 4096 10.1 / 15.1; of 14336 x 4096 25.9 / 20.0;
+        // with most CUs taken by more than 64 rows also a longer K, but for groups of 32
+        // (128 rows of 7168 x 2048, g128 17.7 / 20.1, g64 18.1 / 20.6; 17 rows of 8192 x
+        // 8192 20.8 / 18.0).  Two blocks of 8 waves a CU (of groups of 128 only a full
+        // round has 8): 512 rows of 2048 x 1024 11.4 / 16.1, 128 of 4096 x 4096
+        // 18.3 / 20.8, 48 of 1024 x 8192, g64, 9.4 / 11.1; of 512 columns 128 rows of
+        // N = 4096 9.2 / 7.7; g32 128 of 4096 x 4096 24.9 / 23.5.
+        const uint64_t blocks = (uint64_t)(A.N / 64) * row_tiles16;
+        const bool eight = A.G == 32 || A.G == 64 || A.G == 256 || (A.G == 128 && blocks == 2 * cus);
+        if (blocks <= cus) one_round = A.K <= (4 * blocks > 3 * cus && batch_width > 64 && A.G > 32 ? 8192u : 6144u);
+        else if (2 * blocks >= 3 * cus && blocks <= 2 * cus && eight) one_round = A.K >= 1024 && A.K <= (A.G > 32 ? 4096u : 2048u);
+    } else if (s.layout == 1 && A.K <= 4096 && A.N % 16 == 0) {
+        // 16 columns a block: 17 rows of 1024 x 512 6.3 / 7.7, 64 of 4096 x 1024
+        // 8.3 / 11.5; 32 columns (a full round of them): 32 rows of 4096 x 4096
+        // 9.9 / 13.5; 17 of 6144 x 2048 13.0 / 11.8.
+        const uint64_t blocks = (uint64_t)(A.N / 16) * row_tiles16;
+        one_round = blocks <= cus || (A.N % 32 == 0 && blocks == 2 * cus);
+    }
+    const bool few = s.layout == 0 && A.N % 64 == 0 && batch_width > GEMV_MAX_M && batch_width <= 16 && A.K > 6144 &&
+                     2 * (A.N / 64) <= cus;
     if (((batch_width > 16 && !one_round) || few) && !(s.layout == 1 && (zeros || A.G % 128)) &&
         nh::int4_gemm(ctx, A, nullptr, false, s.layout == 1, strm))
         return nh::check_launch("int4_linear_gemm");
@@ -916,7 +937,7 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
             // CUs have a tile (9216 x 6144 13.0 / 12.2, but 9216 x 8192 13.3 / 14.2,
             // 11008 x 8192 15.7 / 15.3); two rows of 4608 x 4096 9.0 / 8.9, four
             // 9.3 / 9.0.
-            const uint32_t batches = (A.K / 8 + GEMV_ROWS - 1) / GEMV_ROWS, cus = (uint32_t)ctx->cu_count;
+            const uint32_t batches = (A.K / 8 + GEMV_ROWS - 1) / GEMV_ROWS;
             const bool gains = batch_width > 1 || A.K > (2 * tiles >= cus ? 10240u : 6144u);
             const uint32_t most = gains ? std::max(1u, std::min((A.K / 256 + 15) / 16, cus / tiles)) : 1u;
             const uint32_t span = (batches + most - 1) / most, splits = (batches + span - 1) / span;

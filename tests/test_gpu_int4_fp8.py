@@ -302,3 +302,15 @@ def test_int4_linear_tiles(ctx, dev, layout, M, K, N, G, asym):
                              finalize=finalize, aux=aux)
     ok, worst, exact = bf16_close(got[:M], ref, atol=linear_atol(x, gptq_dequant(d), finalize), name="int4 tiles")
     assert ok and exact > 0.9, (worst, exact)
+
+
+# Beside the lines between the 16-row kernels and the tiled form: 16-row GPTQ blocks
+# two a CU (whole rounds of eight waves, and groups of 64 short of one), CT row tiles
+# at 16 and, as a full round, 32 columns a block, and the tiled CT form at the column
+# and row edges that its K > 4096 or its blocks still bring to it.
+@pytest.mark.parametrize("layout,M,K,N,G,asym", [
+    ("gptq", 512, 1024, 1024, 128, False), ("gptq", 400, 1024, 1024, 64, True), ("gptq", 400, 1024, 1024, 128, True),
+    ("ct", 100, 768, 512, 256, False), ("ct", 32, 256, 4096, 128, False), ("ct", 17, 4224, 16, 128, False),
+    ("ct", 49, 4224, 272, 128, False), ("ct", 100, 4352, 1040, 256, False), ("ct", 301, 384, 1040, 128, False)])
+def test_int4_linear_row_lines(ctx, dev, layout, M, K, N, G, asym):
+    test_int4_linear_tiles(ctx, dev, layout, M, K, N, G, asym)
