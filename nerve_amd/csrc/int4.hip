@@ -895,14 +895,14 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
     if (s.layout == 0 && A.N % 64 == 0) {
         // A block a CU: 64 rows of 4096 x 4096 10.1 / 15.1; of 14336 x 4096 25.9 / 20.0;
         // with most CUs taken by more than 64 rows also a longer K, but for groups of 32
-        // (128 rows of 7168 x 2048, g128 17.7 / 20.1, g64 18.1 / 20.6; 17 rows of 8192 x
-        // 8192 20.8 / 18.0).  Two blocks of 8 waves a CU (of groups of 128 only a full
+        // (7168 x 2048, 96 rows 15.6 / 17.4, 128 rows 17.7 / 20.1, g64 18.1 / 20.6; 17
+        // rows of 8192 x 8192 20.8 / 18.0).  Two blocks of 8 waves a CU (of groups of 128 only a full
         // round has 8): 512 rows of 2048 x 1024 11.4 / 16.1, 128 of 4096 x 4096
         // 18.3 / 20.8, 48 of 1024 x 8192, g64, 9.4 / 11.1; of 512 columns 128 rows of
         // N = 4096 9.2 / 7.7; g32 128 of 4096 x 4096 24.9 / 23.5.
         const uint64_t blocks = (uint64_t)(A.N / 64) * row_tiles16;
         const bool eight = A.G == 32 || A.G == 64 || A.G == 256 || (A.G == 128 && blocks == 2 * cus);
-        if (blocks <= cus) one_round = A.K <= (4 * blocks > 3 * cus && batch_width > 64 && A.G > 32 ? 8192u : 6144u);
+        if (blocks <= cus) one_round = A.K <= (4 * blocks >= 3 * cus && batch_width > 64 && A.G > 32 ? 8192u : 6144u);
         else if (2 * blocks >= 3 * cus && blocks <= 2 * cus && eight) one_round = A.K >= 1024 && A.K <= (A.G > 32 ? 4096u : 2048u);
     } else if (s.layout == 1 && A.K <= 4096 && A.N % 16 == 0) {
         // 16 columns a block: 17 rows of 1024 x 512 6.3 / 7.7, 64 of 4096 x 1024

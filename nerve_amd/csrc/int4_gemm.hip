@@ -404,7 +404,12 @@ void launch_seg(const GemmArgs& P, uint32_t mt, hipStream_t st) {
 // more for every MiB of partial sums.  Measured (us, this choice / the other):
 // 64 rows of 14336 x 4096, 16 splits / 28: 20.6 / 22.5; 301 rows of the same,
 // 6 / 3: 65.9 / 81; 300 rows of 4096 x 14336, 3 row tiles / 4: 59.6 / 66; 512
-// rows, 4 / 3: 70 / 92.
+// rows, 4 / 3: 70 / 92.  Two blocks on a CU that hold fewer than six
+// stages times row tiles each cost more than the estimate's 1.2 (CT, two such a CU
+// / one: 33 rows of 8192 x 1024 15.8 / 12.8, 64 of 4096 x 4096 21.0 / 17.9, 128 of
+// 3072 x 3072 19.1 / 17.3; but 17 of 8192 x 8192 with two row tiles 23.6 / 28.8)
+// and are not taken, except where one row group reads the weights (8 rows of 8192 x
+// 8192, g32, 16.8 / 19.2).
 struct Plan {
     uint32_t mt, tgroups, splits;
 };
@@ -420,6 +425,7 @@ Plan plan_gemm(uint32_t M, uint32_t N, uint32_t K, uint32_t tiles, uint32_t cus)
         for (uint32_t splits = 1; splits <= most; splits++) {
             const uint64_t nb = (uint64_t)tiles * tgroups * splits, full = nb / (2 * cus), rem = nb % (2 * cus);
             if (splits > 1 && nb > 2 * cus) break;
+            if (splits > 1 && tgroups > 1 && nb > cus && mt * ((nst + splits - 1) / splits) < 6) continue;
             const double rounds = 1.2 * (double)full + (rem == 0 ? 0.0 : rem <= cus ? 1.0 : 1.2);
             double cost = rounds * ((nst + splits - 1) / splits + 2) * (mt + 2) / 6.0;
             if (splits > 1) cost += 2.5 + 0.25 * splits * (double)bytes / (1 << 20);
