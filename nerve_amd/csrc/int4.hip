@@ -806,8 +806,8 @@ void launch_i8_shape(const PpArgs& P, bool paired, bool ct, uint32_t j, uint32_t
     if (j == 4) {
         if (P.L.B <= 4) launch_i8_form<1, 4, 8, 8, SEG, 1>(P, paired, ct, splits, part, st);
         else if (mt == 1) launch_i8_form<1, 4, 8, 8, SEG>(P, paired, ct, splits, part, st);
-        else if (mt == 3) launch_i8_form<3, 4, 8, 4, SEG>(P, paired, ct, splits, part, st);
-        else launch_i8_form<2, 4, 8, 4, SEG>(P, paired, ct, splits, part, st);
+        else if (mt == 2) launch_i8_form<2, 4, 8, 4, SEG>(P, paired, ct, splits, part, st);
+        else if constexpr (SEG != 2) launch_i8_form<3, 4, 8, 4, SEG>(P, paired, ct, splits, part, st);
     } else {
         if (P.L.B <= 4) launch_i8_form<1, 1, 8, 16, SEG, 1>(P, paired, ct, splits, part, st);
         else if (mt == 1) launch_i8_form<1, 1, 8, 16, SEG>(P, paired, ct, splits, part, st);
@@ -841,7 +841,7 @@ bool launch_i8(const PpArgs& P, bool paired, bool ct, bool one_group, const nerv
     }
     if (mt > 3 || (mt == 3 && j == 1)) return false;
     float* part = splits > 1 ? static_cast<float*>(ctx->split) : nullptr;
-    // (three token tiles and two-block segments spill 47 registers)
+    // (three token tiles and two-block segments spill 47 registers: no such form)
     const uint32_t bpg = A.G % 128 == 0 ? 4 : A.G % 64 == 0 && mt < 3 ? 2 : 1;
     if (bpg == 4) launch_i8_shape<4>(P, paired, ct, j, mt, splits, part, st);
     else if (bpg == 2) launch_i8_shape<2>(P, paired, ct, j, mt, splits, part, st);
