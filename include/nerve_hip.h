@@ -76,7 +76,8 @@ const char* nerve_hip_last_error(void);
 
 /* Opens a context on a HIP device ordinal.  Replaces the Vulkan device handle
  * the reference mounts kernels on (runtime-rs/src/vulkan_compute/
- * compute_device_dispatch.rs:2-249). */
+ * compute_device_dispatch.rs:2-249).  A context takes 32 MiB of device memory for
+ * the INT4 linears' split-K sums at once, its other workspace on demand. */
 nerve_hip_status nerve_hip_open(int device_ordinal, nerve_hip_ctx** out);
 
 /* Releases the context and its workspace.  NULL is accepted. */
@@ -358,9 +359,11 @@ nerve_hip_status nerve_hip_int4_moe_down(nerve_hip_ctx* ctx, const char* spec, c
  * comp.template:85-233; grammar nerve/model_package_shader_templates.py:
  * 3148-3215): per group, the bf16 MFMA sum of (code - 8) x, then
  * fma(group_sum, scale, acc), any batch_width (the CT layout with group % 128
- * != 0 returns NERVE_HIP_UNSUPPORTED).  More than 16 rows may split K over the
- * launch: the partial sums use a part of the context's device memory allocated
- * by nerve_hip_open (32 MiB; no call grows it, so a first call may be captured). */
+ * != 0 returns NERVE_HIP_UNSUPPORTED).  A call of any batch_width may split K
+ * over the launch and then adds the partial sums in a second one: they lie in the
+ * context's 32 MiB of split-K memory (nerve_hip_open allocates it and no call grows
+ * it, so a first call may be captured).  Calls on one context must not overlap
+ * (other streams, parallel graph branches): they share that memory. */
 nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char* spec,
                                        const void* x_bf16, const void* qweight,
                                        const void* scales, const void* zeros,
@@ -406,7 +409,9 @@ nerve_hip_status nerve_hip_silu_multiply_quantize_int8_pairpacked(nerve_hip_ctx*
  * (linear_prequant_int4_gptq.comp.template:65-103, linear_prequant_int4_ct.
  * comp.template:66-108): q in column order (the unpaired quantizer), sums
  * unused (NULL), block_dot = sum_k q (code - 8); the CT layout takes qweight
- * u32 [N, K/8] and scales [N, K/G]. */
+ * u32 [N, K/8] and scales [N, K/G].  A call of any batch_width may split K as
+ * nerve_hip_int4_linear does, through the same memory: calls on one context must
+ * not overlap. */
 nerve_hip_status nerve_hip_int4_linear_pairpacked(nerve_hip_ctx* ctx, const char* spec, const void* q_i8,
                                                  const void* scales_f32, const void* sums_i32,
                                                  const void* qweight, const void* scales, const void* aux_bf16,

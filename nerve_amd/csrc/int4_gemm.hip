@@ -26,8 +26,9 @@
 // cycles, beside some 300 vector instructions of 4 cycles: 112 to expand the
 // codes, 64 to fold the segment, 60 to stage the rows); leaving out the loads
 // changes it by under 10%.  64 columns a wave halve the LDS operand reads of 32
-// columns (512 rows of 4096 x 14336: 70 against 119 us), 16-row tiles past four
-// spill.  Against the 16-row kernels in int4.hip: 301 rows of 14336 x 4096 (CT)
+// columns (512 rows of 4096 x 14336: 70 against 119 us).  Five row tiles spill
+// throughout; four spill 3 to 10 registers in the CT and int8 forms, which the
+// estimate below does not count.  Against the 16-row kernels in int4.hip: 301 rows of 14336 x 4096 (CT)
 // 397 -> 65 us, 512 rows of 4096 x 14336 (GPTQ) 150 -> 69 us, 64 rows of
 // 14336 x 4096 25.9 -> 20.0 us.
 #include <algorithm>
