@@ -342,7 +342,7 @@ def int4_gemv(args, ctx, dev):
     gbs = alg / (kms * 1e-3) / 1e9
     out = base_line(args, gbs, "GB/s", ms, "bf16xint4->f32",
                     {"workload": f"int4_gptq_g128_asym_m{M}_k4096_n14336", "weight_copies_rotated": copies})
-    kname = ("int4_gptq_gemv_kernel<16, 128, true, 1u>" if M == 1 else "int4_gptq_gemv_kernel<16, 128, true, 4u>"
+    kname = ("int4_gptq_gemv_kernel<16, 128, true, 1u, false>" if M == 1 else "int4_gptq_gemv_kernel<16, 128, true, 4u, false>"
              if M <= 4 else "int4_gptq_fixed_kernel<16, 4, 4>" if M <= 16 else "int4_gemm_kernel")
     out["roofline"] = {"bound": "hbm", "kernel": kname, "achieved": gbs, "peak": HBM_PEAK_GBS,
                        "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS, "traffic": traffic_for(kname),
@@ -409,11 +409,17 @@ def int4_moe(args, ctx, dev):
     dn_gbs = dn_alg / (dn_ms * 1e-3) / 1e9
     out = base_line(args, B * k / (step_ms * 1e-3), "expert-tokens/s", ms, "bf16xint4->f32",
                     {"workload": f"int4_ct_sparse_moe_b{B}_h3072_i1024_e256_k10_g32"})
-    out["roofline"] = {"bound": "hbm", "kernel": "sparse_tile_kernel (gate_up)", "achieved": gu_gbs,
+    # The library's choice at this geometry: tiles of routes from 8 blocks a CU on.
+    cus, per = torch.cuda.get_device_properties(dev).multi_processor_count, B * k // E
+    tile = "4u, 4u, 256u, 3u" if per < 3 else "8u, 4u, 256u, 2u" if per < 8 else "16u, 8u, 256u, 2u"
+    gu_name, dn_name = (f"sparse_tile_kernel<{gu}, {tile}, true>" if B * k * -(-n // rows) >= 8 * cus
+                        else f"sparse_int4_kernel<{gu}, 32u, false>"
+                        for gu, n, rows in (("true", I, 64), ("false", H, 128)))
+    out["roofline"] = {"bound": "hbm", "kernel": gu_name, "achieved": gu_gbs,
                        "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gu_gbs / HBM_PEAK_GBS,
-                       "traffic": traffic_for("sparse_tile_kernel<true, 4u, 4u, 256u, 3u, true>"),
+                       "traffic": traffic_for(gu_name),
                        "algorithmic_bytes_per_launch": gu_alg, "launch_ms": gu_ms}
-    out["down"] = {"kernel": "sparse_tile_kernel (down)", "hbm_gbs": dn_gbs, "frac": dn_gbs / HBM_PEAK_GBS,
+    out["down"] = {"kernel": dn_name, "hbm_gbs": dn_gbs, "frac": dn_gbs / HBM_PEAK_GBS,
                    "algorithmic_bytes_per_launch": dn_alg, "launch_ms": dn_ms}
     out["step_ms_graph"] = step_ms
     return out

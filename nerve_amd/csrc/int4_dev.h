@@ -79,7 +79,10 @@ constexpr uint32_t ONES_BF16 = 0x3F803F80u;
 // up to 2^121) that sum passes the largest f32 although the result, fma(dot,
 // s_x s_w, sum) in the shader, does not.  The activation scales are therefore
 // taken 2^-11 times (130048 * 2^121 * 2^-11 < 2^128) and the sum 2^11 times at the
-// end; both are exact, so ordinary results keep every bit.
+// end.  Both are exact for activation scales from 2^-115 on (rows whose block
+// maximum is 2^-108 or more), and such results keep every bit; a smaller scale is
+// rounded to a multiple of 2^-138, where the shader rounds s_x s_w to one of 2^-149.
+// 48 rows of a 4096 / 14336 feed-forward 73.0 -> 74.6 us; up to 16 rows no change.
 constexpr float I8_SCALE_DOWN = 0x1p-11f, I8_SCALE_UP = 0x1p11f;
 
 __device__ __forceinline__ void finalize_store(const Int4Args& A, uint32_t t, uint32_t n, float sum) {
