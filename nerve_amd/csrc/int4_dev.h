@@ -117,7 +117,7 @@ __device__ __forceinline__ float dot2_bf16(uint32_t a, uint32_t b, float c) {
 
 namespace nh {
 
-// Tiled split-K form for more than 16 rows (int4_gemm.hip): launches and
+// Tiled split-K form, mostly for more than 16 rows (int4_gemm.hip): launches and
 // returns true when the shape and alignment allow its loads, else false.
 // `i8` is null for bf16 activations.
 bool int4_gemm(const nerve_hip_ctx* ctx, const Int4Args& A, const PpArgs* i8, bool paired, bool ct, hipStream_t st);

@@ -1,5 +1,5 @@
-// INT4 linears for more than 16 rows: a tiled, split-K form of the kernels in
-// int4.hip, for bf16 and for INT8-prequantized activations.
+// INT4 linears, mostly for more than 16 rows: a tiled, split-K form of the kernels
+// in int4.hip, for bf16 and for INT8-prequantized activations.
 //
 // A block (4 waves) owns 16 MT rows and 256 columns over a range of 128-column
 // stages of K; wave w owns columns 64 w .. 64 w + 63.  Weights go from memory

@@ -10,9 +10,9 @@
 // gives bf16(bf16(y) * route_weight).
 //
 // sparse_tile_kernel contracts an expert's weights against a tile of its routes
-// on the matrix cores (further down); sparse_int4_kernel takes the shapes that it
-// does not.  The latter is HBM-bound weight streaming (one activation row per
-// route), so it is organised around keeping 16-byte weight loads in flight:
+// on the matrix cores (further down); sparse_int4_kernel takes the shapes and the
+// small calls that it does not (launch_tiles).  The latter is HBM-bound weight
+// streaming (one activation row per route), so it is organised around keeping 16-byte weight loads in flight:
 //   * a block (4 waves) owns one route position and a tile of output rows;
 //     each wave owns 8 weight rows (gate/up: 4 gate + the 4 matching up rows;
 //     down: 8 rows) and issues all of its weight and scale loads of a pass
