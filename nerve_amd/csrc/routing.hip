@@ -106,6 +106,15 @@ __global__ __launch_bounds__(64) void topk_kernel(const uint16_t* __restrict__ l
     topk_token(logits + (uint64_t)b * P.E, bias, routes, telemetry, b, true, P, S);
 }
 
+// E <= 64, moe_topk: one wave and block per token.
+__global__ __launch_bounds__(64) void topk_fast_kernel(const uint16_t* __restrict__ logits, const void* __restrict__ bias,
+                                                       uint32_t* __restrict__ routes, uint32_t* __restrict__ telemetry,
+                                                       TopkParams P) {
+    __shared__ __attribute__((aligned(16))) float s_sh[64];
+    const uint32_t b = blockIdx.x;
+    topk_token_fast(logits + (uint64_t)b * P.E, bias, routes, telemetry, b, true, P, nullptr, s_sh);
+}
+
 // E <= 256: one wave per token.  With lds_tel the block counts in LDS (T words, dynamic) and adds its nonzero
 // counts to the telemetry once: popular experts' counters would otherwise take
 // one device atomic per token, all on a few addresses.
@@ -418,11 +427,16 @@ nerve_hip_status nerve_hip_moe_router_topk(nerve_hip_ctx* ctx, const char* spec,
     uint32_t* tel = static_cast<uint32_t*>(telemetry_u32);
     if (ts.experts <= 256) {
         // From 256 tokens on a block takes 16 tokens, so that its LDS counts
-        // are worth their flush (up to 60 KiB of counters).
+        // are worth their flush (up to 60 KiB of counters; 64 experts, top 6, 256
+        // tokens 7.7 -> 7.0 us, 2048 35.8 -> 8.9; with the full softmax 10.7 -> 11.4
+        // and 38.9 -> 13.2).  Below, up to 64 experts take a block per token: four
+        // tokens a block cost 0.3 to 0.7 us (64 experts, 16 tokens 4.2 -> 4.9).
         const uint32_t res = ts.experts + (ts.mode == 1 ? ts.always_count : 0u), T = res + res * (res - 1) / 2;
         const bool lds_tel = tel && batch_width >= 256 && T <= 15360;
         const uint32_t nw = lds_tel ? 16 : 4;
-        topk_wave_kernel<<<(batch_width + nw - 1) / nw, 64 * nw, lds_tel ? T * 4 : 0, strm>>>(
+        if (ts.experts <= 64 && ts.mode == 0 && !lds_tel)
+            topk_fast_kernel<<<batch_width, 64, 0, strm>>>(lg, bias, rt, tel, P);
+        else topk_wave_kernel<<<(batch_width + nw - 1) / nw, 64 * nw, lds_tel ? T * 4 : 0, strm>>>(
             lg, bias, rt, tel, batch_width, lds_tel ? T : 0u, P);
     } else {
         const size_t lds = (size_t)(ts.experts + 3) / 4 * 4 * 8;   // >= E floats rounded up to float4s, twice
