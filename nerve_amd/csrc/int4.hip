@@ -840,6 +840,15 @@ bool launch_i8(const PpArgs& P, bool paired, bool ct, bool one_group, const nerv
         if (splits > 1) j = 4;
     }
     if (mt > 3 || (mt == 3 && j == 1)) return false;
+    // A few rows of a short K, the more with every round of blocks: int4_pp_kernel's
+    // lanes are done with their columns in a shorter chain than blocks of 8 waves are
+    // placed, loaded and summed (us, int4_pp_kernel / here: one row of 512 x 512 3.1 / 4.0,
+    // of 512 x 8192 4.3 / 6.0, of CT 512 x 32768 5.5 / 21.3; two rows of CT 2048 x 32768
+    // 27.7 / 34.8, but of 1024 x 2048 6.2 / 3.9 and five of CT 1536 x 32768 42.3 / 33.4).
+    // Rows in column order, which it brings into nibble order first, gain half as much.
+    const uint32_t blocks = j == 4 ? wide : A.N / 16 * tg, rounds = std::min(8u, (blocks + cus - 1) / cus);
+    const uint64_t chain = (uint64_t)A.B * (A.K < 128 ? 256 : std::max(A.K, 512u) * (paired || ct ? 1 : 2));
+    if (chain <= (A.B == 1 && (ct || rounds >= 4) ? 1300u : ct ? 720u : 640u) * rounds) return false;
     float* part = splits > 1 ? static_cast<float*>(ctx->split) : nullptr;
     // (three token tiles and two-block segments spill 47 registers: no such form)
     const uint32_t bpg = A.G % 128 == 0 ? 4 : A.G % 64 == 0 && mt < 3 ? 2 : 1;

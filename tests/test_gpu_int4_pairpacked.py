@@ -258,3 +258,22 @@ def test_int4_linear_prequant_large_rows(ctx, dev, kind, M, K, N, G):
     assert np.all(np.isfinite(wl.bf16_bits_to_f32(ref)))
     ok, worst, exact = bf16_close(to_np(y, np.uint16), ref, atol=linear_atol(x, gptq_dequant(d)), name="prequant large")
     assert ok and exact > 0.9, (worst, exact)
+
+
+# Few rows on both sides of the line between a lane per column and the matrix cores:
+# one row of K = 640 (CT: 1280) and the next K beyond it, the same with two rounds of
+# blocks, one token per lane group in wide tiles with a wave whose batch runs past K,
+# K = 64, and eight rounds of CT blocks.
+@pytest.mark.parametrize("kind", ["paired", "gptq", "ct"])
+@pytest.mark.parametrize("M,K,N,G", [(1, 640, 96, 64), (1, 704, 96, 64), (1, 1280, 80, 128), (1, 1408, 80, 128),
+                                     (2, 448, 8256, 64), (2, 640, 5120, 128), (3, 640, 5120, 128), (4, 64, 5120, 32),
+                                     (6, 64, 5120, 64), (3, 512, 32784, 128), (10, 512, 32784, 128), (12, 512, 32784, 128)])
+def test_int4_linear_prequant_few_rows(ctx, dev, kind, M, K, N, G):
+    test_int4_linear_prequant_tiles(ctx, dev, kind, M, K, N, G)
+
+
+# Rows near bf16's limit with one token per lane group (K long enough for it).
+@pytest.mark.parametrize("kind", ["paired", "gptq", "ct"])
+@pytest.mark.parametrize("M,K,N,G", [(1, 1536, 96, 128), (4, 1024, 8256, 64)])
+def test_int4_linear_prequant_large_rows_few(ctx, dev, kind, M, K, N, G):
+    test_int4_linear_prequant_large_rows(ctx, dev, kind, M, K, N, G)
