@@ -911,14 +911,28 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
         // N = 4096 9.2 / 7.7; g32 128 of 4096 x 4096 24.9 / 23.5.
         const uint64_t blocks = (uint64_t)(A.N / 64) * row_tiles16;
         const bool eight = A.G == 32 || A.G == 64 || A.G == 256 || (A.G == 128 && blocks == 2 * cus);
-        if (blocks <= cus) one_round = A.K <= (4 * blocks >= 3 * cus && batch_width > 64 && A.G > 32 ? 8192u : 6144u);
-        else if (2 * blocks >= 3 * cus && blocks <= 2 * cus && eight) one_round = A.K >= 1024 && A.K <= (A.G > 32 ? 4096u : 2048u);
+        if (blocks <= cus) {
+            one_round = A.K <= (4 * blocks >= 3 * cus && batch_width > 64 && A.G > 32 ? 8192u : 6144u);
+        } else if (blocks <= 2 * cus) {
+            // Short of one and a half blocks a CU: g64, 80 rows of 2048 x 4096 10.5 / 12.5,
+            // 350 of 1536 x 1024 9.4 / 13.1, of 3072 x 1024 14.6 / 15.9, 300 14.5 / 14.0;
+            // g32, 80 of 1024 x 4096 10.4 / 11.3, 300 of 2048 x 1024 13.7 / 12.8.
+            const bool most = 2 * blocks >= 3 * cus || (A.G == 64 && A.K <= 2048) || (A.G == 32 && A.K <= 1536);
+            one_round = eight && most && A.K >= 1024 && A.K <= (A.G > 32 ? 4096u : 2048u);
+        } else if (blocks <= 3 * cus && A.G <= 128) {
+            // Three blocks a CU: 300 rows of 2048 x 2048 13.0 / 14.2, g64 13.7 / 16.5, 200 of
+            // 2048 x 3072 13.3 / 16.1, g64 14.0 / 18.0; of 1536 x 3072 12.3 / 13.1, g64
+            // 12.8 / 14.5, but 300 of 1536 x 2048 12.1 / 11.4; g64 of 1024 x 2048 11.8 / 10.1.
+            one_round = A.K <= 2560 && A.K >= (A.G == 64 ? 1536u : 1792u);
+        }
     } else if (s.layout == 1 && A.K <= 4096 && A.N % 16 == 0) {
         // 16 columns a block: 17 rows of 1024 x 512 6.3 / 7.7, 64 of 4096 x 1024
         // 8.3 / 11.5; 32 columns (a full round of them): 32 rows of 4096 x 4096
-        // 9.9 / 13.5; 17 of 6144 x 2048 13.0 / 11.8.
+        // 9.9 / 13.5; 17 of 6144 x 2048 13.0 / 11.8.  A short K leaves a second block's
+        // chain short: 33 rows of 512 x 2048 5.0 / 7.2, of 768 x 2048 6.4 / 8.8.
         const uint64_t blocks = (uint64_t)(A.N / 16) * row_tiles16;
-        one_round = blocks <= cus || (A.N % 32 == 0 && blocks == 2 * cus);
+        one_round = blocks <= cus || (A.N % 32 == 0 && blocks == 2 * cus) ||
+                    (A.K <= 512 && blocks <= 2 * cus) || (A.K <= 768 && 2 * blocks <= 3 * cus);
     }
     const bool few = s.layout == 0 && A.N % 64 == 0 && batch_width > GEMV_MAX_M && batch_width <= 16 && A.K > 6144 &&
                      2 * (A.N / 64) <= cus;
