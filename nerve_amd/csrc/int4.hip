@@ -919,11 +919,13 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
             // g32, 80 of 1024 x 4096 10.4 / 11.3, 300 of 2048 x 1024 13.7 / 12.8.
             const bool most = 2 * blocks >= 3 * cus || (A.G == 64 && A.K <= 2048) || (A.G == 32 && A.K <= 1536);
             one_round = eight && most && A.K >= 1024 && A.K <= (A.G > 32 ? 4096u : 2048u);
-        } else if (blocks <= 3 * cus && A.G <= 128) {
-            // Three blocks a CU: 300 rows of 2048 x 2048 13.0 / 14.2, g64 13.7 / 16.5, 200 of
+        } else if (blocks <= 3 * cus ? A.G == 32 || A.G == 64 || A.G == 128
+                                     : blocks > 4 * cus && blocks <= 5 * cus && (A.G == 64 || A.G == 128)) {
+            // Three blocks a CU, or five: 300 rows of 2048 x 2048 13.0 / 14.2, g64 13.7 / 16.5, 200 of
             // 2048 x 3072 13.3 / 16.1, g64 14.0 / 18.0; of 1536 x 3072 12.3 / 13.1, g64
-            // 12.8 / 14.5, but 300 of 1536 x 2048 12.1 / 11.4; g64 of 1024 x 2048 11.8 / 10.1.
-            one_round = A.K <= 2560 && A.K >= (A.G == 64 ? 1536u : 1792u);
+            // 12.8 / 14.5, 400 of 2048 x 3072 19.3 / 21.2, g64 20.6 / 23.6, but 300 of 1536 x
+            // 2048 12.1 / 11.4; g64 of 1024 x 2048 11.8 / 10.1.
+            one_round = A.K <= 2560 && A.K >= (A.G == 64 && blocks <= 3 * cus ? 1536u : 1792u);
         }
     } else if (s.layout == 1 && A.K <= 4096 && A.N % 16 == 0) {
         // 16 columns a block: 17 rows of 1024 x 512 6.3 / 7.7, 64 of 4096 x 1024
