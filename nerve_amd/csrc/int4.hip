@@ -916,16 +916,19 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
         } else if (blocks <= 2 * cus) {
             // Short of one and a half blocks a CU: g64, 80 rows of 2048 x 4096 10.5 / 12.5,
             // 350 of 1536 x 1024 9.4 / 13.1, of 3072 x 1024 14.6 / 15.9, 300 14.5 / 14.0;
+            // g256, 65 of 1280 x 4096 6.5 / 9.8, 350 of 2816 x 1024 12.1 / 13.5;
             // g32, 80 of 1024 x 4096 10.4 / 11.3, 300 of 2048 x 1024 13.7 / 12.8.
-            const bool most = 2 * blocks >= 3 * cus || (A.G == 64 && A.K <= 2048) || (A.G == 32 && A.K <= 1536);
-            one_round = eight && most && A.K >= 1024 && A.K <= (A.G > 32 ? 4096u : 2048u);
-        } else if (blocks <= 3 * cus ? A.G == 32 || A.G == 64 || A.G == 128
-                                     : blocks > 4 * cus && blocks <= 5 * cus && (A.G == 64 || A.G == 128)) {
+            const bool most = 2 * blocks >= 3 * cus || (A.G == 64 && A.K <= 2048) || (A.G == 32 && A.K <= 1536) ||
+                              (A.G == 256 && A.K <= 3072);
+            one_round = eight && most && A.K >= 1024 && A.K <= (A.G > 32 ? 4096u : 2304u);
+        } else if (blocks <= 3 * cus ? A.G == 32 || A.G == 64 || A.G == 128 || A.G == 256
+                                     : blocks > 4 * cus && blocks <= 5 * cus && (A.G == 64 || A.G == 128 || A.G == 256)) {
             // Three blocks a CU, or five: 300 rows of 2048 x 2048 13.0 / 14.2, g64 13.7 / 16.5, 200 of
             // 2048 x 3072 13.3 / 16.1, g64 14.0 / 18.0; of 1536 x 3072 12.3 / 13.1, g64
             // 12.8 / 14.5, 400 of 2048 x 3072 19.3 / 21.2, g64 20.6 / 23.6, but 300 of 1536 x
-            // 2048 12.1 / 11.4; g64 of 1024 x 2048 11.8 / 10.1.
-            one_round = A.K <= 2560 && A.K >= (A.G == 64 && blocks <= 3 * cus ? 1536u : 1792u);
+            // 2048 12.1 / 11.4; g64 of 1024 x 2048 11.8 / 10.1; g256, 256 of 2816 x 3072
+            // 17.5 / 20.7, 65 of 1792 x 8192 11.3 / 13.6.
+            one_round = A.K <= (A.G == 256 ? 2816u : 2560u) && A.K >= (A.G == 64 && blocks <= 3 * cus ? 1536u : 1792u);
         }
     } else if (s.layout == 1 && A.K <= 4096 && A.N % 16 == 0) {
         // 16 columns a block: 17 rows of 1024 x 512 6.3 / 7.7, 64 of 4096 x 1024

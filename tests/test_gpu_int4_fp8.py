@@ -316,11 +316,12 @@ def test_int4_linear_row_lines(ctx, dev, layout, M, K, N, G, asym):
     test_int4_linear_tiles(ctx, dev, layout, M, K, N, G, asym)
 
 
-# More than a round: GPTQ blocks short of one and a half a CU (groups of 64), three and
-# five a CU, CT row tiles two a CU with a short K and the first K beyond it.
+# More than a round: GPTQ blocks short of one and a half a CU (groups of 64 and 256),
+# three and five a CU, CT row tiles two a CU with a short K and the first K beyond it.
 @pytest.mark.parametrize("layout,M,K,N,G,asym", [
     ("gptq", 350, 1024, 1024, 64, True), ("gptq", 350, 1024, 1024, 128, False), ("gptq", 300, 1792, 2048, 128, True),
-    ("gptq", 300, 1536, 2048, 64, False), ("gptq", 400, 1792, 2688, 128, False), ("ct", 33, 512, 2048, 128, False), ("ct", 33, 768, 2048, 256, False),
-    ("ct", 49, 768, 2048, 128, False), ("ct", 33, 896, 2048, 128, False)])
+    ("gptq", 300, 1536, 2048, 64, False), ("gptq", 400, 1792, 2688, 128, False),
+    ("gptq", 350, 1280, 1024, 256, True), ("gptq", 300, 1792, 2048, 256, False),
+    ("ct", 33, 512, 2048, 128, False), ("ct", 33, 768, 2048, 256, False), ("ct", 49, 768, 2048, 128, False), ("ct", 33, 896, 2048, 128, False)])
 def test_int4_linear_more_rounds(ctx, dev, layout, M, K, N, G, asym):
     test_int4_linear_tiles(ctx, dev, layout, M, K, N, G, asym)
