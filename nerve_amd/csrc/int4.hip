@@ -895,12 +895,12 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
     // More than 16 rows: the tiled split-K form, which expands the weights once per
     // 64 rows instead of once per 16; from five rows on also where column tiles are
     // few and K is long (16 rows of 14336 x 4096: 25.4 -> 14.6 us).  The 16-row
-    // kernels stay where one round of their blocks covers the linear and K is short
+    // kernels stay where few rounds of their blocks cover the linear and K is short
     // enough for the launch that adds the split sums to count (us, 16-row kernel /
     // tiled form).
     const uint32_t cus = (uint32_t)ctx->cu_count;
     const uint64_t row_tiles16 = (batch_width + 15) / 16;
-    bool one_round = false;
+    bool few_rounds = false;
     if (s.layout == 0 && A.N % 64 == 0) {
         // A block a CU: 64 rows of 4096 x 4096 10.1 / 15.1; of 14336 x 4096 25.9 / 20.0;
         // with most CUs taken by more than 64 rows also a longer K, but for groups of 32
@@ -908,11 +908,12 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
         // rows of 8192 x 8192 20.8 / 18.0).  Two blocks of 8 waves a CU (of groups of 128 only a full
         // round has 8): 512 rows of 2048 x 1024 11.4 / 16.1, 128 of 4096 x 4096
         // 18.3 / 20.8, 48 of 1024 x 8192, g64, 9.4 / 11.1; of 512 columns 128 rows of
-        // N = 4096 9.2 / 7.7; g32 128 of 4096 x 4096 24.9 / 23.5.
+        // N = 4096 9.2 / 7.7; g32 128 of 4096 x 4096 24.9 / 23.5, of
+        // 2304 x 4096 17.1 / 18.8.
         const uint64_t blocks = (uint64_t)(A.N / 64) * row_tiles16;
         const bool eight = A.G == 32 || A.G == 64 || A.G == 256 || (A.G == 128 && blocks == 2 * cus);
         if (blocks <= cus) {
-            one_round = A.K <= (4 * blocks >= 3 * cus && batch_width > 64 && A.G > 32 ? 8192u : 6144u);
+            few_rounds = A.K <= (4 * blocks >= 3 * cus && batch_width > 64 && A.G > 32 ? 8192u : 6144u);
         } else if (blocks <= 2 * cus) {
             // Short of one and a half blocks a CU: g64, 80 rows of 2048 x 4096 10.5 / 12.5,
             // 350 of 1536 x 1024 9.4 / 13.1, of 3072 x 1024 14.6 / 15.9, 300 14.5 / 14.0;
@@ -920,7 +921,7 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
             // g32, 80 of 1024 x 4096 10.4 / 11.3, 300 of 2048 x 1024 13.7 / 12.8.
             const bool most = 2 * blocks >= 3 * cus || (A.G == 64 && A.K <= 2048) || (A.G == 32 && A.K <= 1536) ||
                               (A.G == 256 && A.K <= 3072);
-            one_round = eight && most && A.K >= 1024 && A.K <= (A.G > 32 ? 4096u : 2304u);
+            few_rounds = eight && most && A.K >= 1024 && A.K <= (A.G > 32 ? 4096u : 2304u);
         } else if (blocks <= 3 * cus ? A.G == 32 || A.G == 64 || A.G == 128 || A.G == 256
                                      : blocks > 4 * cus && blocks <= 5 * cus && (A.G == 64 || A.G == 128 || A.G == 256)) {
             // Three blocks a CU, or five: 300 rows of 2048 x 2048 13.0 / 14.2, g64 13.7 / 16.5, 200 of
@@ -928,7 +929,7 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
             // 12.8 / 14.5, 400 of 2048 x 3072 19.3 / 21.2, g64 20.6 / 23.6, but 300 of 1536 x
             // 2048 12.1 / 11.4; g64 of 1024 x 2048 11.8 / 10.1; g256, 256 of 2816 x 3072
             // 17.5 / 20.7, 65 of 1792 x 8192 11.3 / 13.6.
-            one_round = A.K <= (A.G == 256 ? 2816u : 2560u) && A.K >= (A.G == 64 && blocks <= 3 * cus ? 1536u : 1792u);
+            few_rounds = A.K <= (A.G == 256 ? 2816u : 2560u) && A.K >= (A.G == 64 && blocks <= 3 * cus ? 1536u : 1792u);
         }
     } else if (s.layout == 1 && A.K <= 4096 && A.N % 16 == 0) {
         // 16 columns a block: 17 rows of 1024 x 512 6.3 / 7.7, 64 of 4096 x 1024
@@ -936,12 +937,12 @@ extern "C" nerve_hip_status nerve_hip_int4_linear(nerve_hip_ctx* ctx, const char
         // 9.9 / 13.5; 17 of 6144 x 2048 13.0 / 11.8.  A short K leaves a second block's
         // chain short: 33 rows of 512 x 2048 5.0 / 7.2, of 768 x 2048 6.4 / 8.8.
         const uint64_t blocks = (uint64_t)(A.N / 16) * row_tiles16;
-        one_round = blocks <= cus || (A.N % 32 == 0 && blocks == 2 * cus) ||
+        few_rounds = blocks <= cus || (A.N % 32 == 0 && blocks == 2 * cus) ||
                     (A.K <= 512 && blocks <= 2 * cus) || (A.K <= 768 && 2 * blocks <= 3 * cus);
     }
     const bool few = s.layout == 0 && A.N % 64 == 0 && batch_width > GEMV_MAX_M && batch_width <= 16 && A.K > 6144 &&
                      2 * (A.N / 64) <= cus;
-    if (((batch_width > 16 && !one_round) || few) && !(s.layout == 1 && (zeros || A.G % 128)) &&
+    if (((batch_width > 16 && !few_rounds) || few) && !(s.layout == 1 && (zeros || A.G % 128)) &&
         nh::int4_gemm(ctx, A, nullptr, false, s.layout == 1, strm))
         return nh::check_launch("int4_linear_gemm");
     if (s.layout == 0) {
